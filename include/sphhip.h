@@ -695,7 +695,8 @@ typedef struct sph_batch_desc {
                                * momentum kernel: 1, 2 or 4 (density: twice that;
                                * default 2) */
     int32_t cells_per_block;  /* destination cells each block of the list count
-                               * pass walks: 1..64 (default 1) */
+                               * pass walks: 1..64 (default 0: runs sized by the
+                               * library) */
     void *work;        /* device workspace of sph_batch_workspace_size bytes */
     int64_t work_bytes;
     int32_t *status;   /* device */

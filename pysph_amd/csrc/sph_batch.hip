@@ -1078,7 +1078,7 @@ int batch_lists(sph_ctx *ctx, const sph_batch_desc *d, const BatchWork &w)
                               d->y, d->z, w.perm, w.cell_start, w.cells, ncell_dev,
                               d->max_cells, n, d->radius_scale, d->maxch, w.counts, w.slice_off,
                               w.indices, d->list_cap, d->status, d->pairs, trash,
-                              d->cells_per_block > 0 ? d->cells_per_block : 1);
+                              d->cells_per_block);
     return rc;
 }
 

@@ -1050,7 +1050,13 @@ extern "C" int sph_gather_sorted(sph_ctx *ctx, int64_t n, const int32_t *perm,
 #define MAXSEG 64      // stencil cells handled per batch (27 for d = 1)
 
 #define NN_MAXCH 16    // candidate chunks (of 64) whose hit masks the count pass keeps
-#define NN_CELL_GRID (1 << 20)  // blocks of the count pass (one cell at a time each)
+#define NN_CELL_GRID (1 << 20)  // most blocks of the count pass, cells_per_block given
+// blocks of the count pass by default: enough to balance cells of uneven
+// size over the 6,144 wavefronts the device holds, few enough that a block's
+// run shares its first lookups (100^3 lattice, 74,088 cells: 229 us at 16,384
+// blocks, 204 at 32,768, 217 at 65,536; 256 drops, 941,000 cells: 1,105,
+// 957 and 1,008 us)
+#define NN_COUNT_BLOCKS 32768
 #define NN_OVF_GRID 2048    // blocks of the per-cell fill of flagged cells
 
 struct CellArgs {
@@ -1096,7 +1102,7 @@ struct CellArgs {
     int32_t *ovf_list;
     int32_t *novf;
     // destination cells per block of the count pass (its grid is the cell
-    // count over this, at most NN_CELL_GRID blocks)
+    // count over this, at most NN_CELL_GRID blocks), or 0: NN_COUNT_BLOCKS
     int cells_per_block;
     // device-side plain builds: the fill also writes totals = {slots, nnz,
     // status} (and sets the status bits) from its first thread
@@ -1220,26 +1226,23 @@ template <> __device__ __forceinline__ const float *srec_of<float>(const CellArg
     return a.srec32;
 }
 
-// one destination cell w (one wavefront); seg_start, seg_end, dsts are the
-// block's LDS arrays
-template <bool FILL, typename T>
-__device__ void nnps_cell(const CellArgs &a, int64_t w, int32_t *__restrict__ counts,
-                          const int64_t *__restrict__ slice_off, int32_t *__restrict__ indices,
-                          int32_t *seg_start, int32_t *seg_end, typename Quad<T>::type *dsts)
+// The grid, cell coordinates and stencil reach of destination cell w, shared
+// by the count pass and the fill of flagged cells.
+struct CellBox {
+    int x0, y0, z0, nx, ny, nz, nst, dist;
+};
+
+__device__ __forceinline__ GridDev cell_grid(const CellArgs &a, int32_t key, int32_t ds)
 {
-    const T *drec = drec_of<T>(a);
-    const T *srec = srec_of<T>(a);
-    const int lane = threadIdx.x;
-    const int32_t key = a.dcells[w];
-    if (key == a.trash) return;  // rows stay empty
-    // no source cell within reach: every row of the cell stays empty (counts
-    // start at 0) -- most fluid cells against a wall array
-    if (!FILL && a.s_near && !a.s_near[key]) return;
-    const int32_t ds = a.dstart[key], de = a.dstart[key + 1];
-    const GridDev g =
-        a.grids ? a.grids[a.key_sim ? a.key_sim[key] : a.sim_of[a.dperm[ds]]] : a.g;
-    // the cell's coordinates, recomputed exactly as the binning did (from
-    // the double coordinates it used)
+    return a.grids ? a.grids[a.key_sim ? a.key_sim[key] : a.sim_of[a.dperm[ds]]] : a.g;
+}
+
+// the coordinates of the cell of the destination at sorted position ds,
+// recomputed exactly as the binning did (from the double coordinates it used)
+template <typename T>
+__device__ __forceinline__ void cell_coords(const CellArgs &a, const GridDev &g, int32_t ds,
+                                            int &cx, int &cy, int &cz)
+{
     double c0x, c0y, c0z;
     if (a.ox) {
         const int32_t i0 = a.dperm[ds];
@@ -1247,49 +1250,86 @@ __device__ void nnps_cell(const CellArgs &a, int64_t w, int32_t *__restrict__ co
         c0y = a.oy[i0];
         c0z = a.oz[i0];
     } else {
-        const T *r0 = drec + (int64_t)ds * SPH_REC;
+        const T *r0 = drec_of<T>(a) + (int64_t)ds * SPH_REC;
         c0x = r0[SPH_R_X];
         c0y = r0[SPH_R_Y];
         c0z = r0[SPH_R_Z];
     }
-    const int cx = min(max(cell_coord(c0x, g.cs) - g.cmin0, 0), g.d0 - 1);
-    const int cy = min(max(cell_coord(c0y, g.cs) - g.cmin1, 0), g.d1 - 1);
-    const int cz = min(max(cell_coord(c0z, g.cs) - g.cmin2, 0), g.d2 - 1);
-    // stencil reach: the largest (int)ceil(h*rs/cell) over the cell; a
-    // destination with a smaller reach only sees extra candidates that fail
-    // its distance test, and its own stencil is a sub-box visited in order
-    int dl = 0;
-    for (int32_t t = ds + lane; t < de; t += CW) {
-        double r = (double)drec[(int64_t)t * SPH_REC + SPH_R_H] * a.rs / g.cs;
-        // float h can round up past the h the cell size came from: a reach
-        // of 1 + 1e-7 cells would double the stencil for pairs that only
-        // the float rounding could add
-        if (sizeof(T) == sizeof(float)) r *= 1.0 - 0x1p-20;
-        // bounded so that a non-finite h (rejected on the host, flagged in a
-        // batch) cannot overflow the stencil arithmetic; a reach above 256
-        // cells needs a cell size clamped below radius/256
-        dl = max(dl, r > 0.0 ? (r < 256.0 ? (int)ceil(r) : 256) : 0);
-    }
-    const int dist = wave_max_i(dl);
-    const int x0 = max(cx - dist, 0), x1 = min(cx + dist, g.d0 - 1);
-    const int y0 = max(cy - dist, 0), y1 = min(cy + dist, g.d1 - 1);
-    const int z0 = max(cz - dist, 0), z1 = min(cz + dist, g.d2 - 1);
-    const int nx = x1 - x0 + 1, ny = y1 - y0 + 1, nz = z1 - z0 + 1;
-    const int nst = nx * ny * nz;
-    if (!FILL && !a.same && !a.s_near) {
-        // no source in the stencil: every row of the cell stays empty (counts
-        // start at 0) -- most fluid cells against a wall array.  (A cell's own
-        // array always has its members in the stencil.)
-        int32_t found = 0;
-        for (int sIdx = lane; sIdx < nst; sIdx += CW) {
-            const int iz = sIdx % nz, iy = (sIdx / nz) % ny, ix = sIdx / (nz * ny);
-            const int32_t k = cell_key(g, x0 + ix, y0 + iy, z0 + iz);
-            found |= a.sstart[k + 1] - a.sstart[k];
-        }
-        if (!__builtin_amdgcn_ballot_w64(found != 0)) return;
-    }
+    cx = min(max(cell_coord(c0x, g.cs) - g.cmin0, 0), g.d0 - 1);
+    cy = min(max(cell_coord(c0y, g.cs) - g.cmin1, 0), g.d1 - 1);
+    cz = min(max(cell_coord(c0z, g.cs) - g.cmin2, 0), g.d2 - 1);
+}
 
-    int nchunks = 0;  // chunks per destination over all stencil batches
+// (int)ceil(radius / cell) of one destination: its stencil reach
+template <typename T>
+__device__ __forceinline__ int dest_reach(const CellArgs &a, const GridDev &g, T h)
+{
+    double r = (double)h * a.rs / g.cs;
+    // float h can round up past the h the cell size came from: a reach
+    // of 1 + 1e-7 cells would double the stencil for pairs that only
+    // the float rounding could add
+    if (sizeof(T) == sizeof(float)) r *= 1.0 - 0x1p-20;
+    // bounded so that a non-finite h (rejected on the host, flagged in a
+    // batch) cannot overflow the stencil arithmetic; a reach above 256
+    // cells needs a cell size clamped below radius/256
+    return r > 0.0 ? (r < 256.0 ? (int)ceil(r) : 256) : 0;
+}
+
+__device__ __forceinline__ CellBox cell_box(const GridDev &g, int cx, int cy, int cz, int dist)
+{
+    CellBox b;
+    b.dist = dist;
+    b.x0 = max(cx - dist, 0);
+    b.y0 = max(cy - dist, 0);
+    b.z0 = max(cz - dist, 0);
+    b.nx = min(cx + dist, g.d0 - 1) - b.x0 + 1;
+    b.ny = min(cy + dist, g.d1 - 1) - b.y0 + 1;
+    b.nz = min(cz + dist, g.d2 - 1) - b.z0 + 1;
+    b.nst = b.nx * b.ny * b.nz;
+    return b;
+}
+
+// key of stencil cell s (x outer, y, z inner)
+__device__ __forceinline__ int32_t box_key(const GridDev &g, const CellBox &b, int s)
+{
+    const int iz = s % b.nz, iy = (s / b.nz) % b.ny, ix = s / (b.nz * b.ny);
+    return cell_key(g, b.x0 + ix, b.y0 + iy, b.z0 + iz);
+}
+
+// the largest reach over a cell's destinations: one with a smaller reach
+// only sees extra candidates that fail its distance test, and its own
+// stencil is a sub-box visited in order
+template <typename T>
+__device__ __forceinline__ int cell_reach(const CellArgs &a, const GridDev &g, int32_t ds,
+                                          int32_t de)
+{
+    const T *drec = drec_of<T>(a);
+    int dl = 0;
+    for (int32_t t = ds + (int)threadIdx.x; t < de; t += CW)
+        dl = max(dl, dest_reach<T>(a, g, drec[(int64_t)t * SPH_REC + SPH_R_H]));
+    return wave_max_i(dl);
+}
+
+// The fill of one flagged destination cell w (one wavefront): the distance
+// tests again, each hit written to its row.  seg_start, seg_end, dsts are
+// the block's LDS arrays.
+template <typename T>
+__device__ void nnps_cell_fill(const CellArgs &a, int64_t w, int32_t *__restrict__ counts,
+                               const int64_t *__restrict__ slice_off,
+                               int32_t *__restrict__ indices, int32_t *seg_start,
+                               int32_t *seg_end, typename Quad<T>::type *dsts)
+{
+    const T *drec = drec_of<T>(a);
+    const T *srec = srec_of<T>(a);
+    const int lane = threadIdx.x;
+    const int32_t key = a.dcells[w];
+    if (key == a.trash) return;  // rows stay empty
+    const int32_t ds = a.dstart[key], de = a.dstart[key + 1];
+    const GridDev g = cell_grid(a, key, ds);
+    int cx, cy, cz;
+    cell_coords<T>(a, g, ds, cx, cy, cz);
+    const CellBox box = cell_box(g, cx, cy, cz, cell_reach<T>(a, g, ds, de));
+    const int nst = box.nst;
     for (int32_t g0 = ds; g0 < de; g0 += CW) {  // destination groups of <= 64
         const int gn = min(CW, de - g0);
         const int32_t my_t = g0 + lane;  // destination owned by this lane
@@ -1302,18 +1342,16 @@ __device__ void nnps_cell(const CellArgs &a, int64_t w, int32_t *__restrict__ co
         }
         const uint64_t realmask = __ballot(mreal);
         // SELL-64: entry k of row t lives at slice_off[t/64] + 64*k + t%64
-        int64_t myaddr = 0;    // FILL: address of entry 0 of my row
-        int32_t mycount = 0;   // entries found so far (COUNT and FILL)
-        int32_t myself = -1;   // FILL: entry holding my own index
-        int32_t mylast = -1;   // FILL: last neighbour written to my row
-        if (FILL && lane < gn) myaddr = slice_off[my_t >> 6] + (my_t & 63);
-        int cidx = 0;          // chunk index over the stencil batches
+        int64_t myaddr = 0;    // address of entry 0 of my row
+        int32_t mycount = 0;   // entries written so far
+        int32_t myself = -1;   // entry holding my own index
+        int32_t mylast = -1;   // last neighbour written to my row
+        if (lane < gn) myaddr = slice_off[my_t >> 6] + (my_t & 63);
         for (int b0 = 0; b0 < nst; b0 += MAXSEG) {  // stencil batches
             const int sIdx = b0 + lane;
             int32_t st = 0, cnt = 0;
             if (lane < MAXSEG && sIdx < nst) {
-                const int iz = sIdx % nz, iy = (sIdx / nz) % ny, ix = sIdx / (nz * ny);
-                const int32_t k = cell_key(g, x0 + ix, y0 + iy, z0 + iz);
+                const int32_t k = box_key(g, box, sIdx);
                 st = a.sstart[k];
                 cnt = a.sstart[k + 1] - st;
             }
@@ -1325,7 +1363,7 @@ __device__ void nnps_cell(const CellArgs &a, int64_t w, int32_t *__restrict__ co
                 seg_end[lane] = incl;
             }
             __syncthreads();
-            for (int c0 = 0; c0 < total; c0 += CW, ++cidx) {
+            for (int c0 = 0; c0 < total; c0 += CW) {
                 const int q = c0 + lane;
                 const bool valid = q < total;
                 int32_t p = 0;
@@ -1338,30 +1376,12 @@ __device__ void nnps_cell(const CellArgs &a, int64_t w, int32_t *__restrict__ co
                     }
                     const int prev = lo > 0 ? seg_end[lo - 1] : 0;
                     p = seg_start[lo] + (q - prev);
-                    if (!FILL && g0 == ds && b0 == 0 && q < a.maxch * CW)
-                        a.cand[w * (a.maxch * CW) + q] = p;
                     const T *sr = srec + (int64_t)p * SPH_REC;
                     sx = sr[SPH_R_X];
                     sy = sr[SPH_R_Y];
                     sz = sr[SPH_R_Z];
                 }
-                uint32_t mlo = 0, mhi = 0;  // count: my destination's hit mask of this chunk
-                if (!FILL) {
-                    // every lane runs this loop (EXEC is full): the hit mask
-                    // of destination d is the ballot of the compare, kept in
-                    // lane d with v_writelane (no per-lane select)
-                    const uint64_t validm = __builtin_amdgcn_ballot_w64(valid);
-                    for (int d = 0; d < gn; ++d) {
-                        if (!((realmask >> d) & 1)) continue;  // non-LocalReal: empty row
-                        const auto D = dsts[d];  // same address in every lane
-                        // cPoint_distance2(src, dst), base/point.pxd:35-37
-                        const T ex = sx - D.x, ey = sy - D.y, ez = sz - D.z;
-                        const T d2 = ex * ex + ey * ey + ez * ez;
-                        const uint64_t mask = __builtin_amdgcn_ballot_w64(d2 < D.w) & validm;
-                        wave_writelane2(mlo, mhi, (uint32_t)mask, (uint32_t)(mask >> 32), d);
-                    }
-                }
-                for (int d = 0; FILL && d < gn; ++d) {
+                for (int d = 0; d < gn; ++d) {
                     if (!((realmask >> d) & 1)) continue;  // non-LocalReal: empty row
                     const int32_t t = g0 + d;
                     const auto D = dsts[d];  // same address in every lane
@@ -1371,83 +1391,370 @@ __device__ void nnps_cell(const CellArgs &a, int64_t w, int32_t *__restrict__ co
                     const bool hit = valid && d2 < D.w;
                     const uint64_t mask = __ballot(hit);
                     if (mask == 0) continue;
-                    {
-                        const int nh = __popcll(mask);
-                        const int64_t addr0 = wave_bcast_i64(myaddr, d);
-                        const int32_t k0 = __builtin_amdgcn_readlane(mycount, d);
-                        const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-                        if (hit)  // the slice's lines fill up in L2 from several cells
-                            indices[addr0 + ((int64_t)(k0 + __popcll(mask & below)) << 6)] = p;
-                        const int lastlane = 63 - __clzll(mask);
-                        const int32_t lastp = __builtin_amdgcn_readlane(p, lastlane);
-                        const uint64_t selfm = __ballot(a.same && hit && p == t);
-                        if (lane == d) {
-                            if (selfm) {
-                                const int sl = __ffsll((long long)selfm) - 1;
-                                const uint64_t bsl = sl == 0 ? 0ull : (~0ull >> (64 - sl));
-                                myself = k0 + __popcll(mask & bsl);
-                            }
-                            mycount = k0 + nh;
-                            mylast = lastp;
+                    const int nh = __popcll(mask);
+                    const int64_t addr0 = wave_bcast_i64(myaddr, d);
+                    const int32_t k0 = __builtin_amdgcn_readlane(mycount, d);
+                    const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+                    if (hit)  // the slice's lines fill up in L2 from several cells
+                        indices[addr0 + ((int64_t)(k0 + __popcll(mask & below)) << 6)] = p;
+                    const int lastlane = 63 - __clzll(mask);
+                    const int32_t lastp = __builtin_amdgcn_readlane(p, lastlane);
+                    const uint64_t selfm = __ballot(a.same && hit && p == t);
+                    if (lane == d) {
+                        if (selfm) {
+                            const int sl = __ffsll((long long)selfm) - 1;
+                            const uint64_t bsl = sl == 0 ? 0ull : (~0ull >> (64 - sl));
+                            myself = k0 + __popcll(mask & bsl);
                         }
+                        mycount = k0 + nh;
+                        mylast = lastp;
                     }
                 }
-                if (!FILL) {
-                    mycount += __popc(mlo) + __popc(mhi);
-                    if (cidx < a.maxch && lane < gn)
-                        a.masks[(int64_t)cidx * a.mstride + my_t] = ((uint64_t)mhi << 32) | mlo;
+            }
+        }
+        if (lane < gn && a.same && myself >= 0 && myself < mycount - 1) {
+            // keep the particle itself at the last index (nnps.pyx:612-619)
+            indices[myaddr + ((int64_t)myself << 6)] = mylast;
+            indices[myaddr + ((int64_t)(mycount - 1) << 6)] = my_t;
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// The count pass on the matrix cores.
+//
+// A destination's hits among 64 candidates are the signs of
+//     d^2 - R^2 = |c|^2 - 2 c.d + (|d|^2 - R^2),
+// a contraction of K = 4 per (candidate, destination): row (x, y, z, |c|^2)
+// of the candidate times column (-2x, -2y, -2z, 1) of the destination, plus
+// a constant per destination.  v_mfma_f32_16x16x4_f32 gives 16 candidates x
+// 16 destinations in 32 cycles of the matrix unit, where the FP64 test takes
+// nine FP64 instructions (about 50 issue cycles) per 64 candidates and one
+// destination.
+//
+// The signs are exact: coordinates are taken relative to the destination
+// cell's centre (double subtraction), rounded to float and scaled to cells,
+// and a value within NN_BAND of zero is decided by the reference's own FP64
+// (or float) predicate.  With every coordinate below M = reach + 1 cells the
+// partial sums stay below 3.25 M^2: eight float roundings of them (four
+// products and four additions, in any order), three of |c|^2, one of the
+// constant and two of each coordinate move the value by less than
+// 44 * 2^-24 M^2.  The band is 64 * 2^-24 M^2 (1.5e-5 cells^2: one 64 x 16
+// tile in 150 of a disordered set holds such a pair).  A chunk with a
+// coordinate outside M (a particle clamped into the grid, a non-finite one)
+// is decided by the predicate throughout.
+//
+// Candidate 16 g + 4 b + r of a chunk is row 4 g + r of product b, so lane
+// 16 g + j ends with 16 consecutive candidates of destination j: its signs,
+// shifted together, are a quarter of the destination's 64-bit hit mask.
+//
+// Measured, FP64 test per candidate -> this: 100^3 lattice (14 destinations
+// and 372 candidates a cell) 302 -> 204 us, the 1M dam break's two builds
+// 337 -> 235 us, 256 drops of 6.4M particles in 2D (7 and 61) 1,140 -> 957
+// us.  What is left is the work around the products: with the tile loop
+// skipped the lattice's count takes 135 us, with the chunk loop skipped 61
+// us -- chains of dependent loads and LDS round trips per cell and chunk,
+// which six wavefronts per SIMD (NN_COUNT_WAVES) hide in part.  Eight spill
+// (260 us); counting neighbouring cells together, loading the next cell's or
+// the next chunk's data ahead cost the registers of two wavefronts and were
+// slower on the 3D cells (220 to 250 us).
+#define NN_WIN 512                   // candidates listed in LDS at a time
+#define NN_BAND (64.0f * 0x1p-24f)   // times M^2
+#define NN_FAR 1e30f                 // value of an absent candidate or destination
+
+#define NN_COUNT_WAVES 6              // wavefronts per SIMD the count kernels are compiled for
+
+typedef float nn_f32x4 __attribute__((ext_vector_type(4)));
+
+// Orders one wavefront's LDS accesses among its lanes: the hardware executes
+// them in order, so only the compiler has to be kept from moving them (a
+// __syncthreads would also wait for the wavefront's global stores).
+__device__ __forceinline__ void wave_lds_order()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+struct alignas(16) CountLds {
+    int32_t p[NN_WIN];  // sorted source of each candidate of the window
+    float c[5 * CW];    // the chunk's candidates, 4 floats each; 16 more floats every 16
+    float d[4 * CW];    // the group's destinations (-2x, -2y, -2z, |d|^2 - R^2)
+    int32_t n[4 * CW];  // entries so far: 64 per tile of 16 destinations, a quarter mask's each
+};
+
+// the reference's predicate (cPoint_distance2, base/point.pxd:35-37; nnps.pyx:552)
+template <typename T>
+__device__ __forceinline__ bool nnps_hit(const T *srec, const T *drec, T rs, int32_t p, int32_t t)
+{
+    const T *sr = srec + (int64_t)p * SPH_REC;
+    const T *dr = drec + (int64_t)t * SPH_REC;
+    const T radius = dr[SPH_R_H] * rs;
+    const T ex = sr[SPH_R_X] - dr[SPH_R_X], ey = sr[SPH_R_Y] - dr[SPH_R_Y],
+            ez = sr[SPH_R_Z] - dr[SPH_R_Z];
+    return ex * ex + ey * ey + ez * ez < radius * radius;
+}
+
+// inclusive sum over the wavefront by DPP row shifts and broadcasts (the
+// shuffles of wave_incl_scan_i go through LDS, six round trips in a row)
+__device__ __forceinline__ int wave_incl_scan_dpp(int v)
+{
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);  // row_shr:2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);  // row_shr:4
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);  // row_shr:8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31
+    return v;
+}
+
+// s / n for 0 <= s < 64 and 1 <= n <= 64 without a division: the multiplier
+// is rounded up, and its excess times s stays below 65536 / n
+__device__ __forceinline__ int small_div(int s, int n)
+{
+    const int m = n == 3 ? 21846 : n == 1 ? 65536 : n == 2 ? 32768 : (65535 + n) / n;
+    return (s * m) >> 16;
+}
+
+// hit masks and counts of one destination cell w (one wavefront): its
+// destinations [ds, de), grid and cell coordinates
+template <typename T>
+__device__ __forceinline__ void nnps_cell_count(const CellArgs &a, int64_t w, int32_t ds,
+                                                int32_t de, const GridDev &g, double inv_cs, int cx,
+                                                int cy, int cz, int32_t *__restrict__ counts,
+                                                CountLds &S)
+{
+    const T *drec = drec_of<T>(a);
+    const T *srec = srec_of<T>(a);
+    const int lane = threadIdx.x;
+    // stencil reach: 0 or 1 cells unless a radius exceeds the cell size (the
+    // IEEE quotient radius / cell is above 1 exactly when radius > cell)
+    int dist;
+    {
+        bool any = false, more = false;
+        for (int32_t t = ds + lane; t < de; t += CW) {
+            const double h = (double)drec[(int64_t)t * SPH_REC + SPH_R_H];
+            any |= h > 0.0;
+            more |= h * a.rs > g.cs;
+        }
+        dist = __builtin_amdgcn_ballot_w64(any) != 0;
+        if (__builtin_amdgcn_ballot_w64(more))
+            dist = __builtin_amdgcn_readfirstlane(cell_reach<T>(a, g, ds, de));
+    }
+    const CellBox box = cell_box(g, cx, cy, cz, dist);
+    const int nst = box.nst;
+    const float inv = (float)inv_cs;
+    const double ox = (cx + g.cmin0 + 0.5) * g.cs, oy = (cy + g.cmin1 + 0.5) * g.cs,
+                 oz = (cz + g.cmin2 + 0.5) * g.cs;
+    const float lim = (float)dist + 0.75f;
+    const float band = NN_BAND * (float)((dist + 1) * (dist + 1));
+    const int col = lane & 15, quarter = lane >> 4;  // MFMA column (destination), K index
+    // row `col` of product b, K component `quarter`: candidate 16 (col/4) + 4 b + col%4
+    const int crow = 16 * (col >> 2) + (col & 3);
+    // several lanes list the members of one stencil cell
+    const int sh = nst <= 16 ? 2 : nst <= 32 ? 1 : 0;
+    int nchunks = 0;  // chunks per destination over all stencil batches
+    for (int32_t g0 = ds; g0 < de; g0 += CW) {  // destination groups of <= 64
+        const int gn = min(CW, de - g0);
+        bool odd = false;  // a coordinate outside the band's assumptions
+        float4 dv = make_float4(0.f, 0.f, 0.f, NN_FAR);
+        if (lane < gn && a.dperm[g0 + lane] < a.nd_real) {
+            const T *dr = drec + (int64_t)(g0 + lane) * SPH_REC;
+            const T radius = dr[SPH_R_H] * T(a.rs);
+            const float x = (float)((double)dr[SPH_R_X] - ox) * inv,
+                        y = (float)((double)dr[SPH_R_Y] - oy) * inv,
+                        z = (float)((double)dr[SPH_R_Z] - oz) * inv;
+            odd = !(fmaxf(fmaxf(fabsf(x), fabsf(y)), fabsf(z)) <= lim);
+            const double rr = (double)radius * inv_cs;
+            dv = make_float4(-2.0f * x, -2.0f * y, -2.0f * z,
+                             (float)((double)x * x + (double)y * y + (double)z * z - rr * rr));
+        }
+        wave_lds_order();  // the last group's reads are done
+        *reinterpret_cast<float4 *>(&S.d[4 * lane]) = dv;
+        const bool odd_d = __builtin_amdgcn_ballot_w64(odd) != 0;
+        const int ntiles = (gn + 15) >> 4;
+        for (int t = 0; t < ntiles; ++t) S.n[CW * t + lane] = 0;
+        int cidx = 0;  // chunk index over the stencil batches
+        for (int b0 = 0; b0 < nst; b0 += MAXSEG) {  // stencil batches
+            const int sIdx = b0 + (lane >> sh);
+            int32_t st = 0, n = 0;
+            if (sIdx < nst) {
+                const int r = dist <= 1 ? small_div(sIdx, box.nz) : sIdx / box.nz;
+                const int iz = sIdx - r * box.nz;
+                const int ix = dist <= 1 ? small_div(r, box.ny) : r / box.ny;
+                const int iy = r - ix * box.ny;
+                const int32_t k = cell_key(g, box.x0 + ix, box.y0 + iy, box.z0 + iz);
+                st = a.sstart[k];
+                n = a.sstart[k + 1] - st;
+            }
+            const int sub = lane & ((1 << sh) - 1);
+            const int incl = wave_incl_scan_dpp(sub == 0 ? n : 0);
+            const int total = __builtin_amdgcn_readlane(incl, CW - 1);
+            const int before = incl - n;
+            // no source in the stencil: every row of the cell stays empty
+            // (counts start at 0) -- most fluid cells against a wall array
+            if (total == 0 && nst <= MAXSEG && !a.same) return;
+            for (int w0 = 0; w0 < total; w0 += NN_WIN) {  // windows of candidates
+                wave_lds_order();
+                for (int k = max(0, w0 - before) + sub; k < n && before + k < w0 + NN_WIN;
+                     k += 1 << sh)
+                    S.p[before + k - w0] = st + k;
+                wave_lds_order();
+                const int wn = min(NN_WIN, total - w0);
+                for (int c0 = 0; c0 < wn; c0 += CW, ++cidx) {
+                    const int q = c0 + lane;
+                    float4 v = make_float4(0.f, 0.f, 0.f, NN_FAR);
+                    bool far = false;
+                    if (q < wn) {
+                        const int32_t p = S.p[q];
+                        if (g0 == ds && b0 == 0 && w0 + q < a.maxch * CW)
+                            a.cand[w * (a.maxch * CW) + w0 + q] = p;
+                        const T *sr = srec + (int64_t)p * SPH_REC;
+                        v.x = (float)((double)sr[SPH_R_X] - ox) * inv;
+                        v.y = (float)((double)sr[SPH_R_Y] - oy) * inv;
+                        v.z = (float)((double)sr[SPH_R_Z] - oz) * inv;
+                        far = !(fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fabsf(v.z)) <= lim);
+                        v.w = fmaf(v.x, v.x, fmaf(v.y, v.y, v.z * v.z));
+                    }
+                    const bool all = odd_d || __builtin_amdgcn_ballot_w64(far) != 0;
+                    wave_lds_order();  // the last chunk's reads are done
+                    *reinterpret_cast<float4 *>(&S.c[4 * lane + 16 * (lane >> 4)]) = v;
+                    wave_lds_order();
+                    float A[4];
+#pragma unroll
+                    for (int b = 0; b < 4; ++b)
+                        A[b] = S.c[4 * (crow + 4 * b) + 16 * (crow >> 4) + quarter];
+#pragma unroll 1
+                    for (int t = 0; t < ntiles; ++t) {
+                        const int j = 16 * t + col;
+                        const float C = S.d[4 * j + 3];
+                        const float B = quarter < 3 ? S.d[4 * j + quarter] : 1.0f;
+                        const nn_f32x4 c4 = {C, C, C, C};
+                        nn_f32x4 D[4];
+#pragma unroll
+                        for (int b = 0; b < 4; ++b)
+                            D[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[b], B, c4, 0, 0, 0);
+                        uint32_t bits = 0;
+                        float near = NN_FAR;
+#pragma unroll
+                        for (int e = 15; e >= 0; --e) {
+                            const float x = D[e >> 2][e & 3];
+                            bits = __builtin_amdgcn_alignbit(bits, __float_as_uint(x), 31);
+                            near = __builtin_amdgcn_fmed3f(near, fabsf(x), 0.0f);  // the smaller
+                        }
+                        if (all || __builtin_amdgcn_ballot_w64(near < band)) {
+                            // the undecided pairs by the predicate itself
+                            const int32_t left = wn - (c0 + 16 * quarter);
+                            uint32_t ask = left >= 16 ? 0xffffu : left > 0 ? (1u << left) - 1u : 0u;
+                            if (C == NN_FAR) ask = bits = 0;  // no such destination
+                            if (!all) {
+                                uint32_t in = 0;
+#pragma unroll
+                                for (int e = 15; e >= 0; --e)
+                                    in = 2 * in + (fabsf(D[e >> 2][e & 3]) < band);
+                                ask &= in;
+                            }
+                            while (ask) {
+                                const int e = __ffs(ask) - 1;
+                                ask &= ask - 1;
+                                const bool hit = nnps_hit<T>(srec, drec, T(a.rs),
+                                                             S.p[c0 + 16 * quarter + e], g0 + j);
+                                bits = (bits & ~(1u << e)) | ((uint32_t)hit << e);
+                            }
+                        }
+                        S.n[CW * t + lane] += __popc(bits);
+                        if (cidx < a.maxch && j < gn)
+                            reinterpret_cast<uint16_t *>(a.masks + (int64_t)cidx * a.mstride +
+                                                         g0 + j)[quarter] = (uint16_t)bits;
+                    }
                 }
             }
         }
         nchunks = cidx;
+        wave_lds_order();
         if (lane < gn) {
-            if (!FILL) {
-                counts[my_t] = mycount;
-                a.dcell_of[my_t] = (int32_t)w;
-            } else if (a.same && myself >= 0 && myself < mycount - 1) {
-                // keep the particle itself at the last index (nnps.pyx:612-619)
-                indices[myaddr + ((int64_t)myself << 6)] = mylast;
-                indices[myaddr + ((int64_t)(mycount - 1) << 6)] = my_t;
-            }
+            const int32_t *c = S.n + CW * (lane >> 4) + (lane & 15);  // four quarters
+            counts[g0 + lane] = c[0] + c[16] + c[32] + c[48];
+            a.dcell_of[g0 + lane] = (int32_t)w;
         }
     }
-    if (!FILL && lane == 0) {
+    if (lane == 0) {
         const int ovf = nst > MAXSEG || nchunks > a.maxch;
         a.cell_ovf[w] = ovf ? -1 : nchunks;
         if (ovf) a.ovf_list[atomicAdd(a.novf, 1)] = (int32_t)w;
     }
 }
 
-// FILL = false: every non-empty destination cell (XCD x walks the x-th
-// eighth of the cells with its blocks).  FILL = true: the cells the count
-// pass flagged, listed in a.ovf_list.
-// The count pass of one build over block bid of G: every non-empty destination
-// cell (XCD x walks the x-th eighth of the cells with its blocks; bid is
-// the block's XCD-consistent index, bid % 8 being its XCD).
+// The count pass of one build by block bid of G (one wavefront).  Blocks go
+// round-robin to the XCDs (block b to XCD b % 8): XCD x walks cells
+// [x*ncl/8, (x+1)*ncl/8) with its blocks, each block a contiguous run of
+// them, so every XCD has an equal, contiguous share whatever the grid size
+// (the grid is sized for a bound when the cell count is read on the device).
+// Up to 64 cells of the run are looked up together, one per lane (key,
+// members, grid, cell coordinates): that chain of dependent loads is waited
+// for once per run instead of once per cell.
 template <typename T>
 __device__ __forceinline__ void count_cells(const CellArgs &a, int32_t *__restrict__ counts,
-                                            unsigned bid, unsigned G, int32_t *seg_start,
-                                            int32_t *seg_end, typename Quad<T>::type *dsts)
+                                            unsigned bid, unsigned G, CountLds &S)
 {
     // cells read on the device are bounded by the launch size the scratch
     // was carved for (more cells than that is a status error of the caller,
     // whose lists are then incomplete, never written past)
     int64_t ncl = a.ncell_list;
     if (a.ncell_dev && (int64_t)*a.ncell_dev < ncl) ncl = *a.ncell_dev;
-    // blocks go round-robin to the XCDs (block b to XCD b % 8): XCD x walks
-    // cells [x*ncl/8, (x+1)*ncl/8) with its blocks, so every XCD has an
-    // equal, contiguous share whatever the grid size (the grid is sized for a
-    // bound when the cell count is read on the device)
-    if (G < SPH_NXCD) {  // too few blocks to give every XCD one
-        for (int64_t w = bid; w < ncl; w += G)
-            nnps_cell<false, T>(a, w, counts, nullptr, nullptr, seg_start, seg_end, dsts);
-        return;
+    int64_t lo = 0, hi = ncl;
+    unsigned k = bid, per = G;
+    if (G >= SPH_NXCD) {  // else too few blocks to give every XCD one
+        const unsigned x = bid % SPH_NXCD;
+        k = bid / SPH_NXCD;
+        per = (G - x + SPH_NXCD - 1) / SPH_NXCD;  // blocks on XCD x (>= 1)
+        lo = ncl * x / SPH_NXCD;
+        hi = ncl * (x + 1) / SPH_NXCD;
     }
-    const unsigned x = bid % SPH_NXCD, k = bid / SPH_NXCD;
-    const unsigned per = (G - x + SPH_NXCD - 1) / SPH_NXCD;  // blocks on XCD x (>= 1)
-    const int64_t lo = ncl * x / SPH_NXCD, hi = ncl * (x + 1) / SPH_NXCD;
-    for (int64_t w = lo + k; w < hi; w += per)  // uniform: one wavefront per block
-        nnps_cell<false, T>(a, w, counts, nullptr, nullptr, seg_start, seg_end, dsts);
+    const int64_t run = (hi - lo + per - 1) / per;
+    lo += k * run;
+    if (lo + run < hi) hi = lo + run;
+    const int lane = threadIdx.x;
+    for (int64_t w0 = lo; w0 < hi; w0 += CW) {
+        int32_t ds = 0, de = 0;
+        int cx = 0, cy = 0, cz = 0;
+        GridDev gl = a.g;
+        bool act = w0 + lane < hi;
+        if (act) {
+            const int32_t key = a.dcells[w0 + lane];
+            // particles of void simulations get no rows; nor do cells with no
+            // source cell within reach (most fluid cells against a wall array)
+            act = key != a.trash && !(a.s_near && !a.s_near[key]);
+            if (act) {
+                ds = a.dstart[key];
+                de = a.dstart[key + 1];
+                gl = cell_grid(a, key, ds);
+                cell_coords<T>(a, gl, ds, cx, cy, cz);
+            }
+        }
+        const double inv = 1.0 / gl.cs;
+        uint64_t todo = __builtin_amdgcn_ballot_w64(act);
+        while (todo) {
+            const int l = __ffsll((unsigned long long)todo) - 1;
+            todo &= todo - 1;
+            GridDev g = a.g;
+            if (a.grids) {
+                g.cs = wave_bcast(gl.cs, l);
+                g.cmin0 = __builtin_amdgcn_readlane(gl.cmin0, l);
+                g.cmin1 = __builtin_amdgcn_readlane(gl.cmin1, l);
+                g.cmin2 = __builtin_amdgcn_readlane(gl.cmin2, l);
+                g.d0 = __builtin_amdgcn_readlane(gl.d0, l);
+                g.d1 = __builtin_amdgcn_readlane(gl.d1, l);
+                g.d2 = __builtin_amdgcn_readlane(gl.d2, l);
+                g.key_base = __builtin_amdgcn_readlane(gl.key_base, l);
+                g.tab = nullptr;  // a batch's grids are keyed linearly
+            }
+            nnps_cell_count<T>(a, w0 + l, __builtin_amdgcn_readlane(ds, l),
+                               __builtin_amdgcn_readlane(de, l), g, wave_bcast(inv, l),
+                               __builtin_amdgcn_readlane(cx, l),
+                               __builtin_amdgcn_readlane(cy, l),
+                               __builtin_amdgcn_readlane(cz, l), counts, S);
+        }
+    }
 }
 
 // the rows of the cells the count pass flagged (listed in a.ovf_list), by
@@ -1462,43 +1769,42 @@ __device__ __forceinline__ void fill_flagged(const CellArgs &a, int32_t *__restr
     if (a.status && slice_off[a.nslices] > a.cap) return;  // no room: nothing is written
     const int32_t nov = *a.novf;
     for (int32_t k = bid; k < nov; k += G)
-        nnps_cell<true, T>(a, a.ovf_list[k], counts, slice_off, indices, seg_start, seg_end,
-                           dsts);
+        nnps_cell_fill<T>(a, a.ovf_list[k], counts, slice_off, indices, seg_start, seg_end, dsts);
 }
 
-// FILL = false: the count pass (count_cells).  FILL = true: the cells the
-// count pass flagged (fill_flagged).
-template <bool FILL, typename T>
+template <typename T>
+__global__ void __launch_bounds__(CW) __attribute__((amdgpu_waves_per_eu(NN_COUNT_WAVES)))
+    k_nnps_count(CellArgs a, int32_t *__restrict__ counts)
+{
+    __shared__ CountLds S;
+    count_cells<T>(a, counts, blockIdx.x, gridDim.x, S);
+}
+
+template <typename T>
 __global__ void __launch_bounds__(CW)
-    k_nnps_cells(CellArgs a, int32_t *__restrict__ counts, const int64_t *__restrict__ slice_off,
-                 int32_t *__restrict__ indices)
+    k_nnps_flagged(CellArgs a, int32_t *__restrict__ counts,
+                   const int64_t *__restrict__ slice_off, int32_t *__restrict__ indices)
 {
     __shared__ int32_t seg_start[MAXSEG];
     __shared__ int32_t seg_end[MAXSEG];  // inclusive prefix of the segment sizes
     __shared__ typename Quad<T>::type dsts[CW];  // (x, y, z, radius^2) of the group's destinations
-    if (FILL) {
-        fill_flagged<T>(a, counts, slice_off, indices, blockIdx.x, gridDim.x, seg_start, seg_end,
-                        dsts);
-    } else {
-        count_cells<T>(a, counts, blockIdx.x, gridDim.x, seg_start, seg_end, dsts);
-    }
+    fill_flagged<T>(a, counts, slice_off, indices, blockIdx.x, gridDim.x, seg_start, seg_end,
+                    dsts);
 }
 
 // The count passes of two builds in one launch: blocks [0, g0) the first
 // (g0 a multiple of the XCD count, so block indices keep their XCD), the
 // rest the second -- the smaller build fills the larger one's tail.
 template <typename T>
-__global__ void __launch_bounds__(CW)
-    k_nnps_cells_pair(CellArgs a0, int32_t *__restrict__ counts0, CellArgs a1,
+__global__ void __launch_bounds__(CW) __attribute__((amdgpu_waves_per_eu(NN_COUNT_WAVES)))
+    k_nnps_count_pair(CellArgs a0, int32_t *__restrict__ counts0, CellArgs a1,
                       int32_t *__restrict__ counts1, unsigned g0)
 {
-    __shared__ int32_t seg_start[MAXSEG];
-    __shared__ int32_t seg_end[MAXSEG];
-    __shared__ typename Quad<T>::type dsts[CW];
+    __shared__ CountLds S;
     if (blockIdx.x < g0)
-        count_cells<T>(a0, counts0, blockIdx.x, g0, seg_start, seg_end, dsts);
+        count_cells<T>(a0, counts0, blockIdx.x, g0, S);
     else
-        count_cells<T>(a1, counts1, blockIdx.x - g0, gridDim.x - g0, seg_start, seg_end, dsts);
+        count_cells<T>(a1, counts1, blockIdx.x - g0, gridDim.x - g0, S);
 }
 
 // the flagged cells of two builds in one launch (blockIdx.y picks the build)
@@ -2164,7 +2470,8 @@ static int64_t count_grid(const CellArgs &a, int64_t ncell_launch)
 {
     const int cpb = a.cells_per_block > 0 ? a.cells_per_block : 1;
     const int64_t cgrid = (ncell_launch + cpb - 1) / cpb;
-    return cgrid < NN_CELL_GRID ? cgrid : NN_CELL_GRID;
+    const int64_t most = a.cells_per_block > 0 ? NN_CELL_GRID : NN_COUNT_BLOCKS;
+    return cgrid < most ? cgrid : most;
 }
 
 static int nnps_count(sph_ctx *ctx, CellArgs &a, int64_t ncell_launch, int64_t nd_total,
@@ -2179,10 +2486,10 @@ static int nnps_count(sph_ctx *ctx, CellArgs &a, int64_t ncell_launch, int64_t n
     *nnz_dev = slice_sum + a.nslices;
     rc = count_reset(ctx, a, counts, nd_total);
     if (rc) return rc;
-    auto count_kern = a.f32 ? k_nnps_cells<false, float> : k_nnps_cells<false, double>;
+    auto count_kern = a.f32 ? k_nnps_count<float> : k_nnps_count<double>;
     hipLaunchKernelGGL(count_kern, dim3((unsigned)count_grid(a, ncell_launch)), dim3(CW), 0,
-                       ctx->stream, a, counts, (const int64_t *)nullptr, (int32_t *)nullptr);
-    SPH_LAUNCH_CHECK(ctx, "k_nnps_cells<count>");
+                       ctx->stream, a, counts);
+    SPH_LAUNCH_CHECK(ctx, "k_nnps_count");
     return count_slices(ctx, a, counts, slice_off, slice_sum, scan_off, nd_total);
 }
 
@@ -2193,11 +2500,11 @@ static int nnps_fill(sph_ctx *ctx, const CellArgs &a, int64_t ncell_launch, int6
                        dim3(NN_THREADS), 0, ctx->stream, a, nd_total, counts, slice_off, indices,
                        (const int32_t *)nullptr);
     SPH_LAUNCH_CHECK(ctx, "k_nnps_fill_slices");
-    auto fill_kern = a.f32 ? k_nnps_cells<true, float> : k_nnps_cells<true, double>;
+    auto fill_kern = a.f32 ? k_nnps_flagged<float> : k_nnps_flagged<double>;
     const int64_t fill_grid = ncell_launch < NN_OVF_GRID ? ncell_launch : NN_OVF_GRID;
     hipLaunchKernelGGL(fill_kern, dim3((unsigned)fill_grid), dim3(CW), 0, ctx->stream, a,
                        (int32_t *)counts, slice_off, indices);
-    SPH_LAUNCH_CHECK(ctx, "k_nnps_cells<fill>");
+    SPH_LAUNCH_CHECK(ctx, "k_nnps_flagged");
     return SPH_OK;
 }
 
@@ -2489,10 +2796,10 @@ extern "C" int sph_nnps_build_dev_pair(sph_ctx *ctx, const sph_grid *grid,
     SPH_LAUNCH_CHECK(ctx, "k_nnps_reset_pair");
     const unsigned g0 = pair_split(count_grid(j0.a, j0.nd_cells));
     const int64_t g1 = count_grid(j1.a, j1.nd_cells);
-    auto count_kern = j0.a.f32 ? k_nnps_cells_pair<float> : k_nnps_cells_pair<double>;
+    auto count_kern = j0.a.f32 ? k_nnps_count_pair<float> : k_nnps_count_pair<double>;
     hipLaunchKernelGGL(count_kern, dim3((unsigned)(g0 + g1)), dim3(CW), 0, ctx->stream, j0.a,
                        j0.counts, j1.a, j1.counts, g0);
-    SPH_LAUNCH_CHECK(ctx, "k_nnps_cells_pair<count>");
+    SPH_LAUNCH_CHECK(ctx, "k_nnps_count_pair<count>");
     rc = pair_slices(ctx, j0, sum0, scan0, j1, sum1, scan1);
     if (rc) return rc;
     const unsigned f0 = pair_split(sph_blocks(j0.nd_total, NN_THREADS));
@@ -2651,7 +2958,7 @@ int sph_nnps_build_batch(sph_ctx *ctx, const GridDev *grids, const int32_t *sim_
                          int64_t *nnz_acc, int32_t trash, int cells_per_block)
 {
     SPH_REQUIRE(ctx, maxch >= 1 && maxch <= NN_MAXCH, "sph_nnps_build_batch: bad maxch");
-    SPH_REQUIRE(ctx, cells_per_block >= 1, "sph_nnps_build_batch: bad cells_per_block");
+    SPH_REQUIRE(ctx, cells_per_block >= 0, "sph_nnps_build_batch: bad cells_per_block");
     int rc;
     if (n == 0 || max_cells == 0) return nnps_clear(ctx, n, counts, slice_off);
     CellArgs a = cell_args_base();
@@ -3065,7 +3372,7 @@ __global__ void __launch_bounds__(CW) k_varh_cells(CellArgs a, int32_t *__restri
     __shared__ typename Quad<T>::type dsts[CW];
     int64_t ncl = a.ncell_list;
     if (a.ncell_dev && (int64_t)*a.ncell_dev < ncl) ncl = *a.ncell_dev;
-    // XCD x walks cells [x*ncl/8, (x+1)*ncl/8) with its blocks (k_nnps_cells)
+    // XCD x walks cells [x*ncl/8, (x+1)*ncl/8) with its blocks (count_cells)
     const unsigned G = gridDim.x;
     if (G < SPH_NXCD) {
         for (int64_t w = blockIdx.x; w < ncl; w += G)
