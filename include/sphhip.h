@@ -366,7 +366,11 @@ int sph_nnps_export(sph_ctx *ctx, int64_t nd_real, const int32_t *d_rank,
  * rho[nd_total] is written in original order (rho[d_perm[t]]); out_s (may
  * be NULL) receives the same values at out_s[t * out_s_stride].
  * uniform_h = 1 asserts that every destination and source particle has the
- * same h (then (h_i+h_j)/2 == h_i exactly and h_j is not read). */
+ * same h (then (h_i+h_j)/2 == h_i exactly and h_j is not read).
+ * uniform_h = 2 asserts that and that h lies in [2^-100, 2^100]: the FP64
+ * kernels may then take square roots and divisions without the steps for
+ * extreme exponents (the same values).  The float and staged kernels take 2
+ * as 1. */
 int sph_summation_density(sph_ctx *ctx, int dim, int64_t nd_total, int64_t nd_real,
                           const int32_t *d_perm, const int32_t *counts,
                           const int64_t *slice_off, const int32_t *indices,

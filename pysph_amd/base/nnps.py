@@ -370,6 +370,14 @@ class CellManager:
         return bool(self._h_uniform) and all(
             a.version("h") == self._h_versions.get(a.name) for a in self.arrays_to_bin)
 
+    def h_mode(self):
+        """What the operator kernels are told about h (their uniform_h): 0 read
+        it per pair, 1 every h is the same, 2 and it lies in the range where
+        their short square roots and divisions give the IEEE values."""
+        if not self.uniform_h():
+            return 0
+        return 2 if 2.0 ** -100 <= self.grid.min_h <= 2.0 ** 100 else 1
+
     # -- sorted records --------------------------------------------------
     def shadows(self, array, props):
         """The sorted record tensor of `array` with the fields of `props`

@@ -300,6 +300,79 @@ __device__ __forceinline__ T sph_cubic_gfac_fac(T rx, T ry, T rz, T h, T fac, T 
     return val * fac;
 }
 
+// ------------------------------------------------------------------------
+// The same values with fewer operations, for rows whose destination's h
+// (every pair's h) passes sph_short_h.
+//
+// An IEEE FP64 square root or division is a reciprocal estimate, two
+// refinements and a final correction, wrapped in scaling and special-case
+// steps for operands near the ends of the exponent range: 90 and 62 issue
+// cycles of a wavefront, against 50 and 52 without the wrapping (measured on
+// the MI355X, four wavefronts per SIMD).  With h in [2^-100, 2^100] the
+// wrapping never acts where it could change a result:
+//   * r^2 >= 2^-600: no operand of the steps below is scaled by the IEEE
+//     sequences, which then are these steps, so the bits are the same;
+//   * r^2 < 2^-600 (a particle with itself, r = 0): any root of at most
+//     2^-250 gives q <= 2^-150, where W's polynomial is exactly 1 and the
+//     gradient factor is 0 (q <= 1e-14).
+// The gradient's division by h*r takes its reciprocal estimate from the
+// root's refinement (1/r to about 2^-48) times 1/h instead of a reciprocal
+// instruction; one refinement leaves it as close as the IEEE sequence's own.
+// q > 2 needs no test: 2 - q is clamped at 0, and a term of +-0 leaves a sum
+// that started from +0 unchanged.
+// ------------------------------------------------------------------------
+template <typename T> __device__ __forceinline__ bool sph_short_h(T) { return false; }
+template <> __device__ __forceinline__ bool sph_short_h<double>(double h)
+{
+    return h >= 0x1p-100 && h <= 0x1p100;
+}
+
+// sqrt(x), and rinv ~ 1/sqrt(x)
+__device__ __forceinline__ double sph_short_sqrt(double x, double &rinv)
+{
+    const double y = __builtin_amdgcn_rsq(fmax(x, 0x1p-700));
+    double g = x * y, h = 0.5 * y;
+    const double r = fma(-h, g, 0.5);
+    g = fma(g, r, g);
+    h = fma(h, r, h);
+    g = fma(fma(-g, g, x), h, g);
+    rinv = h + h;
+    return fma(fma(-g, g, x), h, g);
+}
+
+// r/h from inv = RN(1/h): see sph_div_inv
+__device__ __forceinline__ double sph_short_q(double r, double h, double inv)
+{
+    const double q0 = r * inv;
+    return fma(fma(-h, q0, r), inv, q0);
+}
+
+// W (sph_cubic_w_fac) and the gradient factor (sph_cubic_gfac_fac) from r^2
+__device__ __forceinline__ double sph_short_w(double r2, double h, double fac, double inv)
+{
+    double ri;
+    const double q = sph_short_q(sph_short_sqrt(r2, ri), h, inv);
+    const double t = fmax(2.0 - q, 0.0);
+    const double val = q > 1.0 ? 0.25 * t * t * t : 1.0 - 1.5 * (q * q) * (1.0 - 0.5 * q);
+    return val * fac;
+}
+
+__device__ __forceinline__ double sph_short_gfac(double r2, double h, double fac, double inv)
+{
+    double ri;
+    const double rab = sph_short_sqrt(r2, ri);
+    const double q = sph_short_q(rab, h, inv);
+    const bool outer = q >= 1.0;
+    const double t = fmax(2.0 - q, 0.0);
+    const double num = outer ? -0.75 * t * t : 3.0 * (0.75 * q - 1.0);
+    const double den = outer ? h * rab : h * h;
+    double y = inv * (outer ? ri : inv);
+    y = fma(y, fma(-den, y, 1.0), y);
+    const double w = num * y;
+    const double v = fma(fma(-den, w, num), y, w);
+    return (q > 1e-14 ? v : 0.0) * fac;
+}
+
 // gradient factor val*fac so that gradW = r * (val*fac)
 __device__ __forceinline__ double sph_cubic_gfac(int dim, double rx, double ry, double rz,
                                                  double h)

@@ -22,6 +22,14 @@
 #ifndef MOM_NT
 #define MOM_NT 4
 #endif
+// the short sequences pay where a few wavefronts wait for their own
+// arithmetic (15,000 fluid particles 75 -> 63 us a launch, 125,000 in 2D 27
+// -> 21 us), with three records in flight; where the gathers set the pace they
+// do not (1M dam break 650 -> 684 us): up to MOM_SMALL destinations
+#ifndef MOM_NT_SHORT
+#define MOM_NT_SHORT 3
+#endif
+#define MOM_SMALL (256 * 1024)
 // waves per SIMD the momentum kernel is compiled for: 3 caps it at 168
 // registers (172 unbounded, which allows 2 waves), with two 8-byte spills
 // outside the neighbour loop; 0.657 -> 0.649 ms on the 1M dam break
@@ -76,11 +84,12 @@ __device__ __forceinline__ void tait_point(const TaitArgs<T> &E, int64_t t, int3
 // SPHRho (rho_term in sph_terms.h)
 // ---------------------------------------------------------------------------
 // one SELL-64 row of SPHRho, summed from 0 in list order
-template <bool UH, typename T>
+template <bool UH, bool SHORT, typename T>
 __device__ __forceinline__ T rho_row(int dim, T xa, T ya, T za, T ha, T facA,
                                      const int32_t *__restrict__ row, int32_t e,
                                      const T *__restrict__ srec, const T *__restrict__ spm)
 {
+    using P = typename Pair<T>::type;
     T nr = T(0.0);
     int32_t k = 0;
     const T invA = sph_inv_for_div(ha);
@@ -96,27 +105,27 @@ __device__ __forceinline__ T rho_row(int dim, T xa, T ya, T za, T ha, T facA,
             j[u] = __builtin_nontemporal_load(row + ((int64_t)(k + u) << 6));
 #pragma unroll
         for (int u = 0; u < DENS_NT; ++u) {
-            const auto *sp = pm2(spm, srec, j[u]);
+            const P *sp = pm2(spm, srec, j[u]);
             a[u] = sp[0];
             b[u] = sp[1];
             hb[u] = UH ? ha : srec[(int64_t)j[u] * SPH_REC + SPH_R_H];
         }
 #pragma unroll
         for (int u = 0; u < DENS_NT; ++u)
-            nr += rho_term<UH, T>(dim, xa, ya, za, ha, facA, a[u], b[u], hb[u], invA);
+            nr += rho_term<UH, T, P, SHORT>(dim, xa, ya, za, ha, facA, a[u], b[u], hb[u], invA);
     }
     for (; k < e; ++k) {
         const int32_t j = __builtin_nontemporal_load(row + ((int64_t)k << 6));
-        const auto *sp = pm2(spm, srec, j);
+        const P *sp = pm2(spm, srec, j);
         const T hb = UH ? ha : srec[(int64_t)j * SPH_REC + SPH_R_H];
-        nr += rho_term<UH, T>(dim, xa, ya, za, ha, facA, sp[0], sp[1], hb, invA);
+        nr += rho_term<UH, T, P, SHORT>(dim, xa, ya, za, ha, facA, sp[0], sp[1], hb, invA);
     }
     return nr;
 }
 
 // EOS: TaitEquation of the same particle follows, from the density just
 // written to its record (the k_tait arithmetic; the caller passes out_s)
-template <bool UH, bool EOS, typename T>
+template <int HM, bool EOS, typename T>
 __global__ void __launch_bounds__(OP_THREADS)
     k_summation_density(int dim, int64_t nd_total, int64_t nd_real,
                         const int32_t *__restrict__ dperm, SrcLists<T> L,
@@ -153,8 +162,8 @@ __global__ void __launch_bounds__(OP_THREADS)
         const T facA = sph_h_dim(ha, dim) * sph_cubic_fac1<T>(dim);
         for (int s = 0; s < L.nsrc; ++s) {
             const int32_t *row = L.indices[s] + L.slice_off[s][t >> 6] + (t & 63);
-            val = val + rho_row<UH, T>(dim, xa, ya, za, ha, facA, row, e[s], L.srec[s],
-                                       L.spm[s]);
+            val = val + rho_row<h_one<HM, T>, h_short<HM, T>, T>(dim, xa, ya, za, ha, facA, row,
+                                                                 e[s], L.srec[s], L.spm[s]);
         }
     }
     rho[i] = val;
@@ -180,10 +189,13 @@ static int summation_density(sph_ctx *ctx, int dim, int64_t nd_total, int64_t nd
     TaitArgs<T> E;
     memset(&E, 0, sizeof(E));
     if (eos) E = *eos;
-    auto kern = eos ? (uniform_h ? k_summation_density<true, true, T>
-                                 : k_summation_density<false, true, T>)
-                    : (uniform_h ? k_summation_density<true, false, T>
-                                 : k_summation_density<false, false, T>);
+    const bool quick = uniform_h == H_SHORT && sizeof(T) == sizeof(double);
+    auto kern = eos ? (quick       ? k_summation_density<H_SHORT, true, T>
+                       : uniform_h ? k_summation_density<H_ONE, true, T>
+                                   : k_summation_density<H_READ, true, T>)
+                    : (quick       ? k_summation_density<H_SHORT, false, T>
+                       : uniform_h ? k_summation_density<H_ONE, false, T>
+                                   : k_summation_density<H_READ, false, T>);
     hipLaunchKernelGGL(kern, dim3(sph_blocks(nd_total, OP_THREADS)),
                        dim3(OP_THREADS), 0, ctx->stream, dim, nd_total, nd_real, d_perm, L,
                        d_rec, accumulate, rho, out_s, out_s_stride, E);
@@ -421,17 +433,18 @@ int sph_tait_records_f32(sph_ctx *ctx, int64_t n, const int32_t *perm, float *re
 // ---------------------------------------------------------------------------
 // one SELL-64 row of MomentumEquation, summed from 0 in list order; dtf is
 // max-reduced over the row.  NT neighbours' records in flight.
-template <bool UH, typename T, int NT>
+template <bool UH, bool SHORT, typename T, int NT>
 __device__ __forceinline__ void mom_row(int dim, const MomDest<T> &D, T alpha, T beta, T eta,
                                         const int32_t *__restrict__ row, int32_t e,
                                         const T *__restrict__ srec, T &dtf, T &nr0, T &nr1,
                                         T &nr2)
 {
+    using P = typename Pair<T>::type;
     int32_t k = 0;
     // NT neighbours' records in flight, then their terms added in list order
     for (; k + NT <= e; k += NT) {
         int32_t j[NT];
-        typename Pair<T>::type s0[NT], s1[NT], s2[NT], s3[NT], s4[NT];
+        P s0[NT], s1[NT], s2[NT], s3[NT], s4[NT];
         T hb[NT];
 #pragma unroll
         for (int u = 0; u < NT; ++u)
@@ -448,19 +461,19 @@ __device__ __forceinline__ void mom_row(int dim, const MomDest<T> &D, T alpha, T
         }
 #pragma unroll
         for (int u = 0; u < NT; ++u)
-            mom_term<UH, T>(dim, D, alpha, beta, eta, s0[u], s1[u], s2[u], s3[u], s4[u], hb[u],
-                            dtf, nr0, nr1, nr2);
+            mom_term<UH, T, P, SHORT>(dim, D, alpha, beta, eta, s0[u], s1[u], s2[u], s3[u],
+                                      s4[u], hb[u], dtf, nr0, nr1, nr2);
     }
     for (; k < e; ++k) {
         const int32_t j = __builtin_nontemporal_load(row + ((int64_t)k << 6));
         const auto *sr = rec2(srec, j);
         const T hb = UH ? D.ha : srec[(int64_t)j * SPH_REC + SPH_R_H];
-        mom_term<UH, T>(dim, D, alpha, beta, eta, sr[0], sr[1], sr[2], sr[3], sr[4], hb, dtf,
-                        nr0, nr1, nr2);
+        mom_term<UH, T, P, SHORT>(dim, D, alpha, beta, eta, sr[0], sr[1], sr[2], sr[3], sr[4],
+                                  hb, dtf, nr0, nr1, nr2);
     }
 }
 
-template <bool UH, typename T>
+template <int HM, int NT, typename T>
 __global__ void __launch_bounds__(OP_THREADS) __attribute__((amdgpu_waves_per_eu(MOM_WAVES)))
     k_momentum(int dim, int64_t nd_total, int64_t nd_real, const int32_t *__restrict__ dperm,
                SrcLists<T> L, const T *__restrict__ drec, T alpha, T beta, T eta,
@@ -512,10 +525,8 @@ __global__ void __launch_bounds__(OP_THREADS) __attribute__((amdgpu_waves_per_eu
         for (int s = 0; s < L.nsrc; ++s) {
             T nr0 = T(0.0), nr1 = T(0.0), nr2 = T(0.0);
             const int32_t *row = L.indices[s] + L.slice_off[s][t >> 6] + (t & 63);
-            // with h read per pair (!UH) four records in flight would spill
-            // registers at 3 waves per SIMD: two
-            mom_row<UH, T, (UH || sizeof(T) == sizeof(float)) ? MOM_NT : 2>(
-                dim, D, alpha, beta, eta, row, e[s], L.srec[s], dtf, nr0, nr1, nr2);
+            mom_row<h_one<HM, T>, h_short<HM, T>, T, NT>(dim, D, alpha, beta, eta, row, e[s],
+                                                         L.srec[s], dtf, nr0, nr1, nr2);
             o0 = o0 + nr0;
             o1 = o1 + nr1;
             o2 = o2 + nr2;
@@ -570,7 +581,14 @@ static int momentum_av(sph_ctx *ctx, int dim, int64_t nd_total, int64_t nd_real,
     if (rc) return rc;
     rc = sph_prho2_sources(ctx, src, sizeof(T) == sizeof(float));
     if (rc) return rc;
-    auto kern = uniform_h ? k_momentum<true, T> : k_momentum<false, T>;
+    // with h read per pair four records in flight would spill registers at 3
+    // waves per SIMD: two (float: four)
+    constexpr int NT_READ = sizeof(T) == sizeof(float) ? MOM_NT : 2;
+    const bool quick = uniform_h == H_SHORT && sizeof(T) == sizeof(double) && nd_total <= MOM_SMALL;
+    constexpr int QUICK = sizeof(T) == sizeof(double) ? H_SHORT : H_ONE;
+    auto kern = quick       ? k_momentum<QUICK, MOM_NT_SHORT, T>
+                : uniform_h ? k_momentum<H_ONE, MOM_NT, T>
+                            : k_momentum<H_READ, NT_READ, T>;
     hipLaunchKernelGGL(kern, dim3(sph_blocks(nd_total, OP_THREADS)), dim3(OP_THREADS), 0,
                        ctx->stream, dim, nd_total, nd_real, d_perm, L, d_rec, T(alpha),
                        T(beta), T(eta), accumulate, ax, ay, az, dt_fac);

@@ -21,6 +21,7 @@ namespace {
 
 template <typename T> struct PairDest {
     T xa, ya, za, ha, facA, wdpA, ma, rhoa, rhoa2, ca, Pa, ua, va, wa;
+    T inv_ha;  // sph_inv_for_div(ha)
 };
 
 template <typename T> struct PairArgs {
@@ -70,7 +71,7 @@ __device__ __forceinline__ bool art_fab(const PairDest<T> &D, const PairArgs<T> 
     return true;
 }
 
-template <int OP, bool AP, bool UH, typename T, typename P>
+template <int OP, bool AP, bool UH, bool SHORT, typename T, typename P>
 __device__ __forceinline__ void pair_term(int dim, const PairDest<T> &D, const PairArgs<T> &A,
                                           const P *s, int32_t o, const double *const *fr,
                                           T &dtf, T &nr0, T &nr1, T &nr2)
@@ -179,7 +180,11 @@ __device__ __forceinline__ void pair_term(int dim, const PairDest<T> &D, const P
                 }
             }
         }
-        const T g = sph_cubic_gfac_fac<T>(rabx, raby, rabz, hab, fac);
+        T g;
+        if constexpr (SHORT)
+            g = sph_short_gfac(rabx * rabx + raby * raby + rabz * rabz, hab, fac, D.inv_ha);
+        else
+            g = sph_cubic_gfac_fac<T>(rabx, raby, rabz, hab, fac);
         nr0 += tmp * (rabx * g);
         nr1 += tmp * (raby * g);
         nr2 += tmp * (rabz * g);
@@ -187,7 +192,7 @@ __device__ __forceinline__ void pair_term(int dim, const PairDest<T> &D, const P
 }
 
 // one SELL-64 row, summed from 0 in list order
-template <int OP, bool AP, bool UH, typename T>
+template <int OP, bool AP, bool UH, bool SHORT, typename T>
 __device__ __forceinline__ void pair_row(int dim, const PairDest<T> &D, const PairArgs<T> &A,
                                          const int32_t *__restrict__ row, int32_t e,
                                          const T *__restrict__ srec,
@@ -214,7 +219,7 @@ __device__ __forceinline__ void pair_row(int dim, const PairDest<T> &D, const Pa
         }
 #pragma unroll
         for (int u = 0; u < PAIR_NT; ++u)
-            pair_term<OP, AP, UH, T>(dim, D, A, s[u], o[u], fr, dtf, nr0, nr1, nr2);
+            pair_term<OP, AP, UH, SHORT, T>(dim, D, A, s[u], o[u], fr, dtf, nr0, nr1, nr2);
     }
     for (; k < e; ++k) {
         const int32_t j = __builtin_nontemporal_load(row + ((int64_t)k << 6));
@@ -223,11 +228,11 @@ __device__ __forceinline__ void pair_row(int dim, const PairDest<T> &D, const Pa
 #pragma unroll
         for (int f = 0; f < 6; ++f) s[f] = (need >> f) & 1u ? sr[f] : P{};
         const int32_t o = frames ? fperm[j] : 0;
-        pair_term<OP, AP, UH, T>(dim, D, A, s, o, fr, dtf, nr0, nr1, nr2);
+        pair_term<OP, AP, UH, SHORT, T>(dim, D, A, s, o, fr, dtf, nr0, nr1, nr2);
     }
 }
 
-template <int OP, bool AP, bool UH, typename T>
+template <int OP, bool AP, int HM, typename T>
 __global__ void __launch_bounds__(PAIR_THREADS)
     k_pair(int dim, int64_t nd_total, int64_t nd_real, const int32_t *__restrict__ dperm,
            SrcLists<T> L, Frames F, const T *__restrict__ drec, PairArgs<T> A, int accumulate,
@@ -277,12 +282,13 @@ __global__ void __launch_bounds__(PAIR_THREADS)
         D.Pa = d5.y;
         D.facA = sph_h_dim(D.ha, dim) * sph_cubic_fac1<T>(dim);
         D.rhoa2 = T(1.0) / (D.rhoa * D.rhoa);
+        D.inv_ha = sph_inv_for_div(D.ha);
         D.wdpA = AP ? sph_cubic_w_fac<T>(A.deltap, T(0.0), T(0.0), D.ha, D.facA) : T(0.0);
         for (int s = 0; s < L.nsrc; ++s) {
             T nr0 = T(0.0), nr1 = T(0.0), nr2 = T(0.0);
             const int32_t *row = L.indices[s] + L.slice_off[s][t >> 6] + (t & 63);
-            pair_row<OP, AP, UH, T>(dim, D, A, row, e[s], L.srec[s], F.perm[s], F.f[s], dtf,
-                                    nr0, nr1, nr2);
+            pair_row<OP, AP, h_one<HM, T>, h_short<HM, T>, T>(
+                dim, D, A, row, e[s], L.srec[s], F.perm[s], F.f[s], dtf, nr0, nr1, nr2);
             o0 = o0 + nr0;
             o1 = o1 + nr1;
             o2 = o2 + nr2;
@@ -300,7 +306,11 @@ int launch_pair(sph_ctx *ctx, int uniform_h, dim3 grid, int dim, int64_t nd_tota
                 const T *drec, const PairArgs<T> &A, int accumulate, double *ax, double *ay,
                 double *az, double *dt_fac)
 {
-    auto kern = uniform_h ? k_pair<OP, AP, true, T> : k_pair<OP, AP, false, T>;
+    // (the wall force takes no root of r)
+    constexpr int BEST = OP == SPH_PAIR_BOUNDARY_FORCE || sizeof(T) == sizeof(float) ? H_ONE : H_SHORT;
+    auto kern = uniform_h == H_SHORT ? k_pair<OP, AP, BEST, T>
+                : uniform_h          ? k_pair<OP, AP, H_ONE, T>
+                                     : k_pair<OP, AP, H_READ, T>;
     hipLaunchKernelGGL(kern, grid, dim3(PAIR_THREADS), 0, ctx->stream, dim, nd_total, nd_real,
                        dperm, L, F, drec, A, accumulate, ax, ay, az, dt_fac);
     SPH_LAUNCH_CHECK(ctx, "k_pair");

@@ -19,9 +19,9 @@
 // list order (SPHFunctionParticle.eval_single, sph_func.pyx:427-441), added
 // to the output (SPHFunction.eval, sph_func.pyx:208-227).
 // ---------------------------------------------------------------------------
-template <bool UH, typename T, typename P>
+template <bool UH, bool SHORT, typename T, typename P>
 __device__ __forceinline__ T rate_term(int dim, T xa, T ya, T za, T ua, T va, T wa, T ha, T facA,
-                                       P s0, P s1, P s2, P s3, T hb)
+                                       T inv, P s0, P s1, P s2, P s3, T hb)
 {
     T hab, fac;
     if (UH || hb == ha) {
@@ -32,7 +32,11 @@ __device__ __forceinline__ T rate_term(int dim, T xa, T ya, T za, T ua, T va, T 
         fac = sph_h_dim(hab, dim) * sph_cubic_fac1<T>(dim);
     }
     const T rabx = xa - s0.x, raby = ya - s0.y, rabz = za - s1.x;
-    const T g = sph_cubic_gfac_fac<T>(rabx, raby, rabz, hab, fac);
+    T g;
+    if constexpr (SHORT)
+        g = sph_short_gfac(rabx * rabx + raby * raby + rabz * rabz, hab, fac, inv);
+    else
+        g = sph_cubic_gfac_fac<T>(rabx, raby, rabz, hab, fac);
     // kernel.gradient: grad = (pa - pb) * (val*fac)
     const T gx = rabx * g, gy = raby * g, gz = rabz * g;
     const T velx = ua - s2.x, vely = va - s2.y, velz = wa - s3.x;
@@ -40,7 +44,7 @@ __device__ __forceinline__ T rate_term(int dim, T xa, T ya, T za, T ua, T va, T 
     return (velx * gx + vely * gy + velz * gz) * s1.y;
 }
 
-template <bool UH, typename T>
+template <int HM, typename T>
 __global__ void __launch_bounds__(RX_THREADS)
     k_density_rate(int dim, int64_t nd_total, int64_t nd_real, const int32_t *__restrict__ dperm,
                    const int32_t *__restrict__ counts, const int64_t *__restrict__ slice_off,
@@ -58,9 +62,11 @@ __global__ void __launch_bounds__(RX_THREADS)
     const auto d0 = dr[0], d1 = dr[1], d2 = dr[2], d3 = dr[3];
     const T ha = drec[t * SPH_REC + SPH_R_H];
     const T facA = sph_h_dim(ha, dim) * sph_cubic_fac1<T>(dim);
-    T nr = T(0.0);
+    const T inv = sph_inv_for_div(ha);
     const int32_t *row = indices + slice_off[t >> 6] + (t & 63);
     const int32_t e = counts[t];
+    T nr = T(0.0);
+    constexpr bool UH = h_one<HM, T>, SHORT = h_short<HM, T>;
     int32_t k = 0;
     for (; k + RX_NT <= e; k += RX_NT) {
         int32_t j[RX_NT];
@@ -80,15 +86,15 @@ __global__ void __launch_bounds__(RX_THREADS)
         }
 #pragma unroll
         for (int u = 0; u < RX_NT; ++u)
-            nr += rate_term<UH, T>(dim, d0.x, d0.y, d1.x, d2.x, d2.y, d3.x, ha, facA, s0[u],
-                                   s1[u], s2[u], s3[u], hb[u]);
+            nr += rate_term<UH, SHORT, T>(dim, d0.x, d0.y, d1.x, d2.x, d2.y, d3.x, ha, facA, inv,
+                                          s0[u], s1[u], s2[u], s3[u], hb[u]);
     }
     for (; k < e; ++k) {
         const int32_t j = __builtin_nontemporal_load(row + ((int64_t)k << 6));
         const auto *sr = rec2(srec, j);
         const T hb = UH ? ha : srec[(int64_t)j * SPH_REC + SPH_R_H];
-        nr += rate_term<UH, T>(dim, d0.x, d0.y, d1.x, d2.x, d2.y, d3.x, ha, facA, sr[0], sr[1],
-                               sr[2], sr[3], hb);
+        nr += rate_term<UH, SHORT, T>(dim, d0.x, d0.y, d1.x, d2.x, d2.y, d3.x, ha, facA, inv,
+                                      sr[0], sr[1], sr[2], sr[3], hb);
     }
     out[i] = (accumulate ? T(out[i]) : T(0.0)) + nr;
 }
@@ -99,9 +105,9 @@ __global__ void __launch_bounds__(RX_THREADS)
 // is divided): nr += (m_b W_ab(h_ab) / rho_ab) (v_b - v_a) eps with
 // rho_ab = 0.5*(rho_b + rho_a).
 // ---------------------------------------------------------------------------
-template <bool UH, typename T, typename P>
+template <bool UH, bool SHORT, typename T, typename P>
 __device__ __forceinline__ void xsph_term(int dim, T xa, T ya, T za, T ua, T va, T wa, T rhoa,
-                                          T ha, T facA, T eps, P s0, P s1, P s2, P s3, P s4,
+                                          T ha, T facA, T inv, T eps, P s0, P s1, P s2, P s3, P s4,
                                           T hb, T &nr0, T &nr1, T &nr2)
 {
     T hab, fac;
@@ -115,14 +121,17 @@ __device__ __forceinline__ void xsph_term(int dim, T xa, T ya, T za, T ua, T va,
     const T rhoab = T(0.5) * (s4.x + rhoa);
     const T vbax = s2.x - ua, vbay = s2.y - va, vbaz = s3.x - wa;  // cPoint_sub(Vb, Va)
     const T mb = s1.y;
-    const T w = sph_cubic_w_fac<T>(xa - s0.x, ya - s0.y, za - s1.x, hab, fac);
+    const T rx = xa - s0.x, ry = ya - s0.y, rz = za - s1.x;
+    T w;
+    if constexpr (SHORT) w = sph_short_w(rx * rx + ry * ry + rz * rz, hab, fac, inv);
+    else w = sph_cubic_w_fac<T>(rx, ry, rz, hab, fac);
     const T temp = mb * w / rhoab;
     nr0 += temp * vbax * eps;
     nr1 += temp * vbay * eps;
     nr2 += temp * vbaz * eps;
 }
 
-template <bool UH, typename T>
+template <int HM, typename T>
 __global__ void __launch_bounds__(RX_THREADS)
     k_xsph(int dim, int64_t nd_total, int64_t nd_real, const int32_t *__restrict__ dperm,
            const int32_t *__restrict__ counts, const int64_t *__restrict__ slice_off,
@@ -143,9 +152,11 @@ __global__ void __launch_bounds__(RX_THREADS)
     const auto d0 = dr[0], d1 = dr[1], d2 = dr[2], d3 = dr[3], d4 = dr[4];
     const T ha = drec[t * SPH_REC + SPH_R_H];
     const T facA = sph_h_dim(ha, dim) * sph_cubic_fac1<T>(dim);
+    const T inv = sph_inv_for_div(ha);
     T nr0 = T(0.0), nr1 = T(0.0), nr2 = T(0.0);
     const int32_t *row = indices + slice_off[t >> 6] + (t & 63);
     const int32_t e = counts[t];
+    constexpr bool UH = h_one<HM, T>, SHORT = h_short<HM, T>;
     int32_t k = 0;
     for (; k + RX_NT <= e; k += RX_NT) {
         int32_t j[RX_NT];
@@ -166,15 +177,15 @@ __global__ void __launch_bounds__(RX_THREADS)
         }
 #pragma unroll
         for (int u = 0; u < RX_NT; ++u)
-            xsph_term<UH, T>(dim, d0.x, d0.y, d1.x, d2.x, d2.y, d3.x, d4.x, ha, facA, eps, s0[u],
-                             s1[u], s2[u], s3[u], s4[u], hb[u], nr0, nr1, nr2);
+            xsph_term<UH, SHORT, T>(dim, d0.x, d0.y, d1.x, d2.x, d2.y, d3.x, d4.x, ha, facA, inv,
+                                    eps, s0[u], s1[u], s2[u], s3[u], s4[u], hb[u], nr0, nr1, nr2);
     }
     for (; k < e; ++k) {
         const int32_t j = __builtin_nontemporal_load(row + ((int64_t)k << 6));
         const auto *sr = rec2(srec, j);
         const T hb = UH ? ha : srec[(int64_t)j * SPH_REC + SPH_R_H];
-        xsph_term<UH, T>(dim, d0.x, d0.y, d1.x, d2.x, d2.y, d3.x, d4.x, ha, facA, eps, sr[0],
-                         sr[1], sr[2], sr[3], sr[4], hb, nr0, nr1, nr2);
+        xsph_term<UH, SHORT, T>(dim, d0.x, d0.y, d1.x, d2.x, d2.y, d3.x, d4.x, ha, facA, inv, eps,
+                                sr[0], sr[1], sr[2], sr[3], sr[4], hb, nr0, nr1, nr2);
     }
     ox[i] = (accumulate ? T(ox[i]) : T(0.0)) + nr0;
     if (oy) oy[i] = (accumulate ? T(oy[i]) : T(0.0)) + nr1;
@@ -205,7 +216,9 @@ static int density_rate(sph_ctx *ctx, int dim, int64_t nd_total, int64_t nd_real
     int rc = check_list_op<T>(ctx, "sph_density_rate", dim, nd_total, nd_real, d_perm, counts,
                               slice_off, d_rec, s_rec, out);
     if (rc || nd_total == 0) return rc;
-    auto kern = uniform_h ? k_density_rate<true, T> : k_density_rate<false, T>;
+    auto kern = uniform_h == H_SHORT ? k_density_rate<H_SHORT, T>
+                : uniform_h          ? k_density_rate<H_ONE, T>
+                                     : k_density_rate<H_READ, T>;
     hipLaunchKernelGGL(kern, dim3(sph_blocks(nd_total, RX_THREADS)), dim3(RX_THREADS), 0,
                        ctx->stream, dim, nd_total, nd_real, d_perm, counts, slice_off, indices,
                        d_rec, s_rec, accumulate, out);
@@ -222,7 +235,12 @@ static int xsph(sph_ctx *ctx, int dim, int64_t nd_total, int64_t nd_real, const 
     int rc = check_list_op<T>(ctx, "sph_xsph", dim, nd_total, nd_real, d_perm, counts,
                               slice_off, d_rec, s_rec, ox);
     if (rc || nd_total == 0) return rc;
-    auto kern = uniform_h ? k_xsph<true, T> : k_xsph<false, T>;
+    // the gathers set the pace of a large array, and the short sequences' longer
+    // live ranges cost more than they save there (512,000 fluid particles 288
+    // us, 317 with them)
+    auto kern = uniform_h == H_SHORT && nd_total <= 256 * 1024 ? k_xsph<H_SHORT, T>
+                : uniform_h          ? k_xsph<H_ONE, T>
+                                     : k_xsph<H_READ, T>;
     hipLaunchKernelGGL(kern, dim3(sph_blocks(nd_total, RX_THREADS)), dim3(RX_THREADS), 0,
                        ctx->stream, dim, nd_total, nd_real, d_perm, counts, slice_off, indices,
                        d_rec, s_rec, T(eps), accumulate, ox, oy, oz);

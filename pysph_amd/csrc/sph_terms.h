@@ -19,6 +19,21 @@ __device__ __forceinline__ const typename Pair<T>::type *rec2(const T *rec, int6
     return reinterpret_cast<const typename Pair<T>::type *>(rec + j * SPH_REC);
 }
 
+// What an operator kernel knows about h, from its caller's uniform_h: H_READ
+// (0: read per pair), H_ONE (1: every h is the same) and H_SHORT (2: and lies
+// in the range of sph_short_h; FP64, the float kernels take it as H_ONE).
+enum { H_READ = 0, H_ONE = 1, H_SHORT = 2 };
+template <int HM, typename T> constexpr bool h_one = HM != H_READ;
+template <int HM, typename T> constexpr bool h_short = HM == H_SHORT && sizeof(T) == sizeof(double);
+
+// whether every active lane's h takes the short sequences (one answer for
+// the wavefront, where the caller does not know)
+template <bool UH, typename T> __device__ __forceinline__ bool short_rows(T h)
+{
+    if constexpr (!UH || sizeof(T) == sizeof(float)) return false;
+    else return !__builtin_amdgcn_ballot_w64(!sph_short_h<T>(h));
+}
+
 // ---------------------------------------------------------------------------
 // SPHRho
 // ---------------------------------------------------------------------------
@@ -26,17 +41,30 @@ __device__ __forceinline__ const typename Pair<T>::type *rec2(const T *rec, int6
 // szm = (z, m) of the source record, hb its h (not read when UH)
 // invA: the destination's sph_inv_for_div(h_a), so q = r/h_a is the IEEE
 // quotient from three operations (sph_div_inv)
-template <bool UH, typename T, typename P>
+// SHORT: short_rows holds; FLAT: every z difference is exactly zero (and adds
+// nothing to r^2)
+template <bool UH, typename T, typename P, bool SHORT = false, bool FLAT = false>
 __device__ __forceinline__ T rho_term(int dim, T xa, T ya, T za, T ha, T facA, P sxy, P szm,
                                       T hb, T invA)
 {
-    // with h_b == h_a, 0.5*(h_a+h_b) == h_a exactly and h_dim(h)*sigma is the
-    // destination's value: reuse it instead of dividing again
-    if (UH || hb == ha)
-        return sph_cubic_w_fac<T>(xa - sxy.x, ya - sxy.y, za - szm.x, ha, facA, invA) * szm.y;
-    const T hab = T(0.5) * (ha + hb);
-    const T fac = sph_h_dim(hab, dim) * sph_cubic_fac1<T>(dim);
-    return sph_cubic_w_fac<T>(xa - sxy.x, ya - sxy.y, za - szm.x, hab, fac) * szm.y;
+    if constexpr (SHORT) {
+        const T rx = xa - sxy.x, ry = ya - sxy.y;
+        T r2 = rx * rx + ry * ry;
+        if constexpr (!FLAT) {
+            const T rz = za - szm.x;
+            r2 = r2 + rz * rz;
+        }
+        return sph_short_w(r2, ha, facA, invA) * szm.y;
+    } else {
+        // with h_b == h_a, 0.5*(h_a+h_b) == h_a exactly and h_dim(h)*sigma is
+        // the destination's value: reuse it instead of dividing again
+        if (UH || hb == ha)
+            return sph_cubic_w_fac<T>(xa - sxy.x, ya - sxy.y, za - szm.x, ha, facA, invA) *
+                   szm.y;
+        const T hab = T(0.5) * (ha + hb);
+        const T fac = sph_h_dim(hab, dim) * sph_cubic_fac1<T>(dim);
+        return sph_cubic_w_fac<T>(xa - sxy.x, ya - sxy.y, za - szm.x, hab, fac) * szm.y;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -50,7 +78,8 @@ template <typename T> struct MomDest {
 // one neighbour term of MomentumEquation (pressure_funcs.pyx:252-391).
 // Source record slots: s0 = (x, y), s1 = (z, m), s2 = (u, v), s3 = (w, P/rho^2),
 // s4 = (rho, cs); hb its h (not read when UH).
-template <bool UH, typename T, typename P>
+// SHORT, FLAT as rho_term; FLAT takes m from s3.x, reads no s1, and leaves nr2
+template <bool UH, typename T, typename P, bool SHORT = false, bool FLAT = false>
 __device__ __forceinline__ void mom_term(int dim, const MomDest<T> &D, T alpha, T beta, T eta,
                                          const P s0, const P s1, const P s2, const P s3,
                                          const P s4, T hb, T &dtf, T &nr0, T &nr1, T &nr2)
@@ -67,17 +96,22 @@ __device__ __forceinline__ void mom_term(int dim, const MomDest<T> &D, T alpha, 
     }
     const T rabx = D.xa - s0.x;
     const T raby = D.ya - s0.y;
-    const T rabz = D.za - s1.x;
     const T vabx = D.ua - s2.x;
     const T vaby = D.va - s2.y;
-    const T vabz = D.wa - s3.x;
-    const T dot = vabx * rabx + vaby * raby + vabz * rabz;
-    const T rab2 = rabx * rabx + raby * raby + rabz * rabz;
+    T dot = vabx * rabx + vaby * raby;
+    T rab2 = rabx * rabx + raby * raby;
+    T rabz = T(0.0);
+    if constexpr (!FLAT) {
+        rabz = D.za - s1.x;
+        const T vabz = D.wa - s3.x;
+        dot = dot + vabz * rabz;
+        rab2 = rab2 + rabz * rabz;
+    }
     const T den = rab2 + eta * eta * hab * hab;
     const T q = hab * dot / den;  // the same quotient as mu below
     const T f = fabs(q);
     dtf = f > dtf ? f : dtf;
-    const T mb = s1.y, rhob = s4.x, cb = s4.y;
+    const T mb = FLAT ? s3.x : s1.y, rhob = s4.x, cb = s4.y;
     // Pb * (1.0/(rhob*rhob)), computed once per source particle (k_prho2)
     T tmp = D.Pa * D.rhoa2 + s3.y;
     // Monaghan viscosity, applied when dot < 0; evaluated for every pair and
@@ -90,10 +124,12 @@ __device__ __forceinline__ void mom_term(int dim, const MomDest<T> &D, T alpha, 
     const T piab = dot < 0 ? pi_v : T(0.0);
     tmp += piab;
     tmp *= -mb;
-    const T g = sph_cubic_gfac_fac<T>(rabx, raby, rabz, hab, fac, inv);
+    T g;
+    if constexpr (SHORT) g = sph_short_gfac(rab2, hab, fac, inv);
+    else g = sph_cubic_gfac_fac<T>(rabx, raby, rabz, hab, fac, inv);
     nr0 += tmp * (rabx * g);
     nr1 += tmp * (raby * g);
-    nr2 += tmp * (rabz * g);
+    if constexpr (!FLAT) nr2 += tmp * (rabz * g);
 }
 
 // ---------------------------------------------------------------------------

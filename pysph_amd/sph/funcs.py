@@ -91,7 +91,7 @@ class SPHRho(CSPHFunctionParticle):
                 ctx.handle, kernel.dim, self.dest.get_number_of_particles(),
                 self.dest.num_real_particles, p(cm.bins[self.dest.name].perm), p(cnt), p(soff),
                 p(idx),
-                p(drec), p(srec), int(cm.uniform_h()), int(bool(accumulate)), p(output1), out_s,
+                p(drec), p(srec), cm.h_mode(), int(bool(accumulate)), p(output1), out_s,
                 REC))
         if name:
             cm.written(self.dest, name, out_s is not None)
@@ -136,7 +136,7 @@ class SPHRho(CSPHFunctionParticle):
                     ctx.handle, ctypes.byref(cm.grid), f0.nbr_locator.radius_scale, kernel.dim,
                     f0.dest.get_number_of_particles(), f0.dest.num_real_particles,
                     p(cm.bins[f0.dest.name].perm), ctypes.byref(src), p(drec),
-                    int(cm.uniform_h()), int(bool(accumulate)), p(output1), out_s, REC))
+                    cm.h_mode(), int(bool(accumulate)), p(output1), out_s, REC))
             if name:
                 cm.written(f0.dest, name, out_s is not None)
             return
@@ -151,7 +151,7 @@ class SPHRho(CSPHFunctionParticle):
             with profiling.region("summation_density"):
                 ctx.check(fn(ctx.handle, kernel.dim, f0.dest.get_number_of_particles(),
                              f0.dest.num_real_particles, p(cm.bins[f0.dest.name].perm),
-                             ctypes.byref(src), p(drec), int(cm.uniform_h()), 0, p(output1),
+                             ctypes.byref(src), p(drec), cm.h_mode(), 0, p(output1),
                              out_s, REC, tf.ro, tf.co, tf.gamma, 0, p(touts[0]), p(touts[1]),
                              p_s, cs_s, prho2_s))
             cm.written(f0.dest, name, True)
@@ -165,7 +165,7 @@ class SPHRho(CSPHFunctionParticle):
         with profiling.region("summation_density"):
             ctx.check(fn(ctx.handle, kernel.dim, f0.dest.get_number_of_particles(),
                          f0.dest.num_real_particles, p(cm.bins[f0.dest.name].perm),
-                         ctypes.byref(src), p(drec), int(cm.uniform_h()),
+                         ctypes.byref(src), p(drec), cm.h_mode(),
                          int(bool(accumulate)), p(output1), out_s, REC))
         if name:
             cm.written(f0.dest, name, out_s is not None)
@@ -298,7 +298,7 @@ class MomentumEquation(SPHFunctionParticle):
                 self.dest.num_real_particles, p(cm.bins[self.dest.name].perm), p(cnt), p(soff),
                 p(idx),
                 p(drec), p(srec), 0 if fresh else cm.bins[self.source.name].n,
-                int(cm.uniform_h()), self.alpha,
+                cm.h_mode(), self.alpha,
                 self.beta, self.eta,
                 int(bool(accumulate)), p(output1), p(output2), p(output3), p(self.d('dt_fac'))))
         if not fresh:
@@ -350,7 +350,7 @@ class MomentumEquation(SPHFunctionParticle):
                     ctx.handle, ctypes.byref(cm.grid), f0.nbr_locator.radius_scale, kernel.dim,
                     f0.dest.get_number_of_particles(), f0.dest.num_real_particles,
                     p(cm.bins[f0.dest.name].perm), ctypes.byref(src), p(drec),
-                    int(cm.uniform_h()), f0.alpha, f0.beta, f0.eta, int(bool(accumulate)),
+                    cm.h_mode(), f0.alpha, f0.beta, f0.eta, int(bool(accumulate)),
                     p(output1), p(output2), p(output3), p(f0.d('dt_fac'))))
         else:
             fn = (ctx.lib.sph_momentum_av_multi_f32 if cm.precision == "single"
@@ -358,7 +358,7 @@ class MomentumEquation(SPHFunctionParticle):
             with profiling.region("momentum_av"):
                 ctx.check(fn(ctx.handle, kernel.dim, f0.dest.get_number_of_particles(),
                              f0.dest.num_real_particles, p(cm.bins[f0.dest.name].perm),
-                             ctypes.byref(src), p(drec), int(cm.uniform_h()), f0.alpha,
+                             ctypes.byref(src), p(drec), cm.h_mode(), f0.alpha,
                              f0.beta, f0.eta, int(bool(accumulate)), p(output1), p(output2),
                              p(output3), p(f0.d('dt_fac'))))
         for f, fr in zip(funcs, fresh):
@@ -412,7 +412,7 @@ def _pair_launch(funcs, kernel, output1, output2, output3, accumulate, names):
     with profiling.region(f0.id):
         ctx.check(fn(ctx.handle, kernel.dim, f0.dest.get_number_of_particles(),
                      f0.dest.num_real_particles, p(cm.bins[f0.dest.name].perm),
-                     ctypes.byref(src), p(drec), int(cm.uniform_h()), ctypes.byref(prm),
+                     ctypes.byref(src), p(drec), cm.h_mode(), ctypes.byref(prm),
                      ctypes.byref(frames) if frames is not None else None,
                      int(bool(accumulate)), p(output1), p(output2), p(output3), p(dt_fac)))
     if uses_prho2:
@@ -625,7 +625,7 @@ class SPHDensityRate(SPHFunctionParticle):
         with profiling.region("density_rate"):
             ctx.check(fn(ctx.handle, kernel.dim, self.dest.get_number_of_particles(),
                          self.dest.num_real_particles, p(cm.bins[self.dest.name].perm), p(cnt),
-                         p(soff), p(idx), p(drec), p(srec), int(cm.uniform_h()),
+                         p(soff), p(idx), p(drec), p(srec), cm.h_mode(),
                          int(bool(accumulate)), p(output1)))
         for name in (names or ()):
             if name:
@@ -665,7 +665,7 @@ class XSPHCorrection(CSPHFunctionParticle):
         with profiling.region("xsph"):
             ctx.check(fn(ctx.handle, kernel.dim, self.dest.get_number_of_particles(),
                          self.dest.num_real_particles, p(cm.bins[self.dest.name].perm), p(cnt),
-                         p(soff), p(idx), p(drec), p(srec), int(cm.uniform_h()), self.eps,
+                         p(soff), p(idx), p(drec), p(srec), cm.h_mode(), self.eps,
                          int(bool(accumulate)), p(output1), p(output2), p(output3)))
         for name in (names or ()):
             if name:
