@@ -697,7 +697,7 @@ typedef struct sph_batch_desc {
                                * particle tiles (default 0: one tile per block) */
     int32_t nbr_tile;         /* neighbour records in flight per lane in the fused
                                * momentum kernel: 1, 2 or 4 (density: twice that;
-                               * default 2) */
+                               * default 4) */
     int32_t cells_per_block;  /* destination cells each block of the list count
                                * pass walks: 1..64 (default 0: runs sized by the
                                * library) */

@@ -22,7 +22,7 @@ import torch
 from .batch import TUNE_FIELDS
 
 SPACE = {
-    "cells_per_block": (1, 2, 4, 8),
+    "cells_per_block": (0, 1, 2, 4, 8),
     "op_threads": (64, 128, 256),
     "op_blocks_per_cu": (0, 4, 8, 16),
     "nbr_tile": (1, 2, 4),
@@ -30,7 +30,7 @@ SPACE = {
     "staged": (0, 1),
 }
 
-DEFAULT = {"cells_per_block": 1, "op_threads": 256, "op_blocks_per_cu": 0, "nbr_tile": 2,
+DEFAULT = {"cells_per_block": 0, "op_threads": 256, "op_blocks_per_cu": 0, "nbr_tile": 4,
            "persistent": 0, "staged": 0}
 
 
