@@ -283,6 +283,14 @@ def ptr(t):
     return t.data_ptr()
 
 
+def _raw_stream(index):
+    """Handle of torch's current stream on device `index`."""
+    return torch.cuda.current_stream(index).cuda_stream
+
+
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", _raw_stream)
+
+
 class Context:
     """One sph_ctx per device, bound to the caller's current torch stream, or
     -- when `stream` is given -- to that torch stream for good (a context of
@@ -298,8 +306,9 @@ class Context:
         self.device_index = idx
         self.fixed_stream = stream is not None
         self.stream = stream if stream is not None else torch.cuda.current_stream(self.device)
+        self.raw_stream = self.stream.cuda_stream
         h = _vp()
-        rc = self.lib.sph_ctx_create(ctypes.byref(h), idx, _vp(self.stream.cuda_stream))
+        rc = self.lib.sph_ctx_create(ctypes.byref(h), idx, _vp(self.raw_stream))
         if rc != SPH_OK:
             raise SphError(rc, f"sph_ctx_create(device={idx}) failed")
         self.handle = h
@@ -308,10 +317,13 @@ class Context:
         """Follow torch's current stream (torch ops and our kernels stay ordered)."""
         if self.fixed_stream:
             return
-        s = torch.cuda.current_stream(self.device)
-        if s.cuda_stream != self.stream.cuda_stream:
-            self.stream = s
+        # the raw handle alone: this runs about eleven times per evaluation,
+        # and a torch.cuda.Stream object costs 5 us each time
+        raw = _raw_stream(self.device_index)
+        if raw != self.raw_stream:
+            s = torch.cuda.current_stream(self.device)
             self.check(self.lib.sph_ctx_set_stream(self.handle, _vp(s.cuda_stream)))
+            self.stream, self.raw_stream = s, s.cuda_stream
 
     def check(self, rc, allow=()):
         if rc == SPH_OK or rc in allow:
@@ -339,8 +351,9 @@ _contexts = {}
 
 def context(device=None):
     """The shared Context for `device` (default cuda:0)."""
-    dev = torch.device(device) if device is not None else torch.device("cuda", 0)
-    key = dev.index if dev.index is not None else 0
+    if device is not None and not isinstance(device, torch.device):
+        device = torch.device(device)
+    key = (device.index if device is not None else None) or 0
     ctx = _contexts.get(key)
     if ctx is None:
         ctx = Context(torch.device("cuda", key))

@@ -56,10 +56,10 @@ class _SharedEvent:
     def __init__(self):
         self.ev = None
 
-    def record(self):
+    def record(self, stream=None):
         if self.ev is None:
             self.ev = torch.cuda.Event()
-            self.ev.record()
+            self.ev.record(stream)
 
     def query(self):
         self.record()
@@ -253,7 +253,9 @@ class CellManager:
         """Record the event of the device-to-host copies queued since the
         last one (after an evaluation's list builds)."""
         if self._open_event is not None:
-            self._open_event.record()
+            # the context's stream is the current one: looking it up again
+            # for the event costs 5 us
+            self._open_event.record(self._ctx().stream)
             self._open_event = None
 
     def _poll_grid_check(self):
@@ -387,10 +389,13 @@ class CellManager:
         # every field asked for so far is refreshed with this one launch, so
         # that one evaluation needs about one gather per array
         wanted = self._wanted.setdefault(array.name, [])
+        fresh, have, now = True, b.shadow_ver, array._version
         for p in props:
             if p not in wanted:
                 wanted.append(p)
-        if any(b.shadow_ver.get(p) != array.version(p) for p in props):
+            if have.get(p) != now.get(p, 0):
+                fresh = False
+        if not fresh:
             # ... except the fields a kernel writes into the records itself
             # (written(shadow_written=True): density and the equation of
             # state), unless asked for now: after a binning their copies
