@@ -238,6 +238,8 @@ _SIGNATURES = {
     "sph_batch_eval": (_i32, [_vp, _vp]),
     "sph_batch_stage": (_i32, [_vp, _vp, _dbl]),
     "sph_batch_vjp": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "sph_batch_rk2_step_kept": (_i32, [_vp, _vp, _dbl, _vp]),
+    "sph_batch_rk2_vjp": (_i32, [_vp, _vp, _dbl, _vp, _vp, _vp, _vp]),
     "sph_fill": (_i32, [_vp, _i64, _dbl, _vp]),
 }
 

@@ -4,11 +4,12 @@ artificial viscosity to a target end state.
 ``Rollout`` advances one simulation (the same kernels as the batched path:
 SPHRho, Tait, MomentumEquation + Monaghan viscosity, PositionStepping, RK2
 of solver/integrator.py:467-498) for ``nsteps`` steps, keeping the positions
-and velocities every ``checkpoint`` steps.  ``Rollout.backward`` walks the
-segments in reverse: it recomputes a segment from its checkpoint, keeping
-each evaluation's neighbour lists and sorted records, and then applies the
-hand-written vector-Jacobian kernels (``sph_batch_vjp``) over those frozen
-lists, stage by stage.  For RK2, X1 = X0 + dt/2 F(X0), X2 = X0 + dt F(X1):
+and velocities every ``checkpoint`` steps, and each evaluation's neighbour
+lists and sorted records in the last segment.  ``Rollout.backward`` walks the
+segments in reverse: it recomputes a segment from its checkpoint (all but the
+one whose evaluations are kept), keeping them likewise, and then applies the
+hand-written vector-Jacobian kernels (``sph_batch_rk2_vjp``) over those frozen
+lists, step by step.  For RK2, X1 = X0 + dt/2 F(X0), X2 = X0 + dt F(X1):
 
     X1bar = J_F(X1)^T (dt X2bar);  X0bar = X2bar + X1bar + J_F(X0)^T (dt/2 X1bar)
 
@@ -52,13 +53,13 @@ class Rollout:
             nb = s.work.numel()
             self.seg_work = [torch.empty(nb, dtype=torch.uint8, device=s.device)
                              for _ in range(2 * self.checkpoint)]
-            self.alpha_bar = torch.zeros(1, dtype=torch.float64, device=s.device)
         self.main_work = (s.desc.work, s.desc.work_bytes)
         for wk in self.seg_work:
             self._use(wk)
             self._call("sph_batch_init_workspace")
         self._use(None)
         self.checkpoints = []
+        self.kept = None  # the segment whose evaluations seg_work holds
         self.alpha = 0.0
 
     # -- pieces ---------------------------------------------------------
@@ -87,15 +88,14 @@ class Rollout:
         self.alpha = float(alpha)
         s.desc.alpha = self.alpha
 
-    def _step(self, works=None):
-        """One RK2 step; evaluation k of it uses works[k] when given."""
-        self._call("sph_batch_save_initial")
-        self._use(works[0] if works else None)
-        self._call("sph_batch_eval")
-        self._call("sph_batch_stage", self.dt / 2)
-        self._use(works[1] if works else None)
-        self._call("sph_batch_eval")
-        self._call("sph_batch_stage", self.dt)
+    def _step(self, j=None):
+        """One RK2 step; with j, its evaluations are kept in the workspaces of
+        step j of a segment."""
+        if j is None:
+            self._call("sph_batch_rk2_step", self.dt)
+            return
+        self._use(self.seg_work[2 * j])
+        self._call("sph_batch_rk2_step_kept", self.dt, self.seg_work[2 * j + 1].data_ptr())
         self._use(None)
 
     # -- forward / backward ---------------------------------------------
@@ -105,14 +105,18 @@ class Rollout:
         s = self.sim
         s.stream.wait_stream(torch.cuda.current_stream(s.device))
         self._set_initial(u0, v0, w0, alpha)
-        self.checkpoints = []
+        self.checkpoints, self.kept = [], None
         keys = self._state_keys()
+        last = (self.nsteps - 1) // self.checkpoint
         for k in range(self.nsteps):
-            if k % self.checkpoint == 0:
+            seg, j = divmod(k, self.checkpoint)
+            if j == 0:
                 with torch.cuda.stream(s.stream):
                     self.checkpoints.append({q: s.t[q].clone() for q in keys})
-            self._step()
+            # the last segment is the first that backward needs: keep it now
+            self._step(j if seg == last else None)
         s.check()
+        self.kept = last
         with torch.cuda.stream(s.stream):
             out = tuple(s.t[q].clone() for q in keys[:self.dim])
         s.synchronize()
@@ -125,56 +129,31 @@ class Rollout:
         s.stream.wait_stream(torch.cuda.current_stream(s.device))
         keys = self._state_keys()
         d = self.dim
-        dt = self.dt
-        vel = keys[d:]
         with torch.cuda.stream(s.stream):  # every tensor op below is ordered with the kernels
-            bar = {q: torch.zeros(self.n, dtype=torch.float64, device=s.device) for q in keys}
-            for c, q in enumerate(keys[:d]):
-                bar[q].copy_(pos_bar[c])
-            out = {q: torch.empty_like(bar[q]) for q in keys}
+            # adjoints of the state, one row per component in the order of keys
+            bar = torch.zeros((2 * d, self.n), dtype=torch.float64, device=s.device)
+            for c in range(d):
+                bar[c].copy_(pos_bar[c])
+            x1bar = torch.empty_like(bar)
             alpha_total = torch.zeros(1, dtype=torch.float64, device=s.device)
             for seg in reversed(range(len(self.checkpoints))):
                 first = seg * self.checkpoint
                 nseg = min(self.checkpoint, self.nsteps - first)
-                for q in keys:
-                    s.t[q].copy_(self.checkpoints[seg][q])
-                for j in range(nseg):
-                    self._step(self.seg_work[2 * j:2 * j + 2])
+                if self.kept != seg:
+                    self.kept = None
+                    for q in keys:
+                        s.t[q].copy_(self.checkpoints[seg][q])
+                    for j in range(nseg):
+                        self._step(j)
+                    self.kept = seg
                 for j in reversed(range(nseg)):
                     # X1bar = J_F(X1)^T (dt X2bar);  X0bar = X2bar + X1bar + J_F(X0)^T (dt/2 X1bar)
-                    x1bar = self._vjp(self.seg_work[2 * j + 1], {q: dt * bar[q] for q in keys},
-                                      out, alpha_total)
-                    add = self._vjp(self.seg_work[2 * j],
-                                    {q: (0.5 * dt) * x1bar[q] for q in keys}, out, alpha_total)
-                    bar = {q: bar[q] + x1bar[q] + add[q] for q in keys}
-            res = tuple(bar[q].clone() for q in vel) + (alpha_total.clone(),)
+                    self._use(self.seg_work[2 * j])
+                    self._call("sph_batch_rk2_vjp", self.dt, self.seg_work[2 * j + 1].data_ptr(),
+                               bar.data_ptr(), x1bar.data_ptr(), alpha_total.data_ptr())
+                    self._use(None)
+            res = tuple(bar[d + c].clone() for c in range(d)) + (alpha_total,)
         s.check()
-        return res
-
-    def _vjp(self, work, fbar, out, alpha_total):
-        """J_F(X)^T fbar for the evaluation kept in `work`; F = (u, a)."""
-        s = self.sim
-        keys = self._state_keys()
-        d = self.dim
-        vel = keys[d:]
-        self._use(work)
-        p = lambda t: t.data_ptr() if t is not None else None
-        abar = [fbar[q] for q in vel]
-        xb = [out[q] for q in keys[:d]]
-        ub = [out[q] for q in vel]
-        s.ctx.check(s.ctx.lib.sph_batch_vjp(
-            s.ctx.handle, ctypes.byref(s.desc), p(abar[0]), p(abar[1]),
-            p(abar[2]) if d == 3 else None, p(xb[0]), p(xb[1]), p(xb[2]) if d == 3 else None,
-            p(ub[0]), p(ub[1]), p(ub[2]) if d == 3 else None, p(self.alpha_bar)))
-        self._use(None)
-        with torch.cuda.stream(s.stream):
-            res = {}
-            for c, q in enumerate(keys[:d]):
-                res[q] = out[q].clone()
-            for c, q in enumerate(vel):
-                # dx/dt = u: the position rows of fbar go to the velocities
-                res[q] = out[q] + fbar[keys[c]]
-            alpha_total += self.alpha_bar
         return res
 
 
