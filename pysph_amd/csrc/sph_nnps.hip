@@ -553,6 +553,7 @@ __global__ void __launch_bounds__(NN_THREADS)
 #define BSCAN_ITEMS 16
 #define BSCAN_TILE (BSCAN_THREADS * BSCAN_ITEMS)
 #define BSCAN_MAX_TILES 2048
+#define BSCAN_DIRECT 4  // tiles up to which k_bin_tile_scan does without k_bin_tile_sums
 
 __global__ void __launch_bounds__(NN_THREADS)
     k_copy_i32(const int32_t *__restrict__ src, int64_t n, int32_t *__restrict__ dst)
@@ -581,17 +582,38 @@ __device__ __forceinline__ int2 bscan_block_sum(int32_t a, int32_t b, int2 *s_pa
     return t;
 }
 
+// a thread's BSCAN_ITEMS counts from base on (0 past nc): counts is 256-byte
+// aligned and base a multiple of BSCAN_ITEMS, so a whole run goes in as int4
+__device__ __forceinline__ void bscan_load(const int32_t *__restrict__ counts, int64_t base,
+                                           int64_t nc, int32_t (&c)[BSCAN_ITEMS])
+{
+    if (base + BSCAN_ITEMS <= nc) {
+#pragma unroll
+        for (int k = 0; k < BSCAN_ITEMS / 4; ++k) {
+            const int4 v = ((const int4 *)(counts + base))[k];
+            c[4 * k] = v.x;
+            c[4 * k + 1] = v.y;
+            c[4 * k + 2] = v.z;
+            c[4 * k + 3] = v.w;
+        }
+        return;
+    }
+#pragma unroll
+    for (int k = 0; k < BSCAN_ITEMS; ++k) c[k] = base + k < nc ? counts[base + k] : 0;
+}
+
 __global__ void __launch_bounds__(BSCAN_THREADS)
     k_bin_tile_sums(const int32_t *__restrict__ counts, int64_t nc, int2 *__restrict__ tile_sum)
 {
     __shared__ int2 s_part[BSCAN_THREADS / 64];
     const int64_t base = (int64_t)blockIdx.x * BSCAN_TILE + (int64_t)threadIdx.x * BSCAN_ITEMS;
+    int32_t c[BSCAN_ITEMS];
+    bscan_load(counts, base, nc, c);
     int32_t a = 0, b = 0;
 #pragma unroll
     for (int k = 0; k < BSCAN_ITEMS; ++k) {
-        const int32_t c = base + k < nc ? counts[base + k] : 0;
-        a += c;
-        b += c > 0;
+        a += c[k];
+        b += c[k] > 0;
     }
     const int2 t = bscan_block_sum(a, b, s_part);
     if (threadIdx.x == 0) tile_sum[blockIdx.x] = t;
@@ -606,28 +628,47 @@ __global__ void __launch_bounds__(BSCAN_THREADS)
     __shared__ int2 s_part[BSCAN_THREADS / 64];
     __shared__ int2 s_wave[BSCAN_THREADS / 64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    // totals of the tiles before this one, eight loads in flight per thread
+    // totals of the tiles before this one, eight loads in flight per thread:
+    // from their sums or, without k_bin_tile_sums, from the counts themselves
     int32_t pa = 0, pb = 0;
-    for (int64_t q0 = 0; q0 < (int64_t)blockIdx.x; q0 += 8 * BSCAN_THREADS) {
-        int2 v[8];
+    if (tile_sum) {
+        for (int64_t q0 = 0; q0 < (int64_t)blockIdx.x; q0 += 8 * BSCAN_THREADS) {
+            int2 v[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int64_t q = q0 + (int64_t)u * BSCAN_THREADS + tid;
-            v[u] = q < (int64_t)blockIdx.x ? tile_sum[q] : make_int2(0, 0);
+            for (int u = 0; u < 8; ++u) {
+                const int64_t q = q0 + (int64_t)u * BSCAN_THREADS + tid;
+                v[u] = q < (int64_t)blockIdx.x ? tile_sum[q] : make_int2(0, 0);
+            }
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                pa += v[u].x;
+                pb += v[u].y;
+            }
         }
+    } else {
+        const int4 *c4 = (const int4 *)counts;
+        const int n4 = (int)blockIdx.x * (BSCAN_TILE / 4);
+        for (int q0 = 0; q0 < n4; q0 += 8 * BSCAN_THREADS) {
+            int4 v[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            pa += v[u].x;
-            pb += v[u].y;
+            for (int u = 0; u < 8; ++u) {
+                const int q = q0 + u * BSCAN_THREADS + tid;
+                v[u] = q < n4 ? c4[q] : make_int4(0, 0, 0, 0);
+            }
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                pa += v[u].x + v[u].y + v[u].z + v[u].w;
+                pb += (v[u].x > 0) + (v[u].y > 0) + (v[u].z > 0) + (v[u].w > 0);
+            }
         }
     }
     const int2 pre = bscan_block_sum(pa, pb, s_part);
     const int64_t base = (int64_t)blockIdx.x * BSCAN_TILE + (int64_t)tid * BSCAN_ITEMS;
     int32_t c[BSCAN_ITEMS];
+    bscan_load(counts, base, nc, c);
     int32_t a = 0, b = 0;
 #pragma unroll
     for (int k = 0; k < BSCAN_ITEMS; ++k) {
-        c[k] = base + k < nc ? counts[base + k] : 0;
         a += c[k];
         b += c[k] > 0;
     }
@@ -729,11 +770,17 @@ int sph_bin_sort(sph_ctx *ctx, int64_t n, int64_t nc, const int32_t *cell_of, in
     int32_t *large = nlarge + 1;
     const int64_t ntiles = (nc + BSCAN_TILE - 1) / BSCAN_TILE;
     if (ntiles <= BSCAN_MAX_TILES) {
-        // starts, the compact list of non-empty cell keys and its count
-        int2 *tile_sum = (int2 *)((char *)ctx->scratch + ((scratch_off + 255) & ~(size_t)255));
-        hipLaunchKernelGGL(k_bin_tile_sums, dim3((unsigned)ntiles), dim3(BSCAN_THREADS), 0,
-                           ctx->stream, slot, nc, tile_sum);
-        SPH_LAUNCH_CHECK(ctx, "k_bin_tile_sums");
+        // starts, the compact list of non-empty cell keys and its count; the
+        // tiles' sums by a launch of their own unless every tile can add up
+        // the counts before it in one or two rounds of loads (3 tiles: 3.8 +
+        // 6.8 -> 5.2 us; at 16 the one launch took 12.3 us, the two 7.9)
+        int2 *tile_sum = nullptr;
+        if (ntiles > BSCAN_DIRECT) {
+            tile_sum = (int2 *)((char *)ctx->scratch + ((scratch_off + 255) & ~(size_t)255));
+            hipLaunchKernelGGL(k_bin_tile_sums, dim3((unsigned)ntiles), dim3(BSCAN_THREADS), 0,
+                               ctx->stream, slot, nc, tile_sum);
+            SPH_LAUNCH_CHECK(ctx, "k_bin_tile_sums");
+        }
         hipLaunchKernelGGL(k_bin_tile_scan, dim3((unsigned)ntiles), dim3(BSCAN_THREADS), 0,
                            ctx->stream, slot, nc, (const int2 *)tile_sum, cell_start, cells,
                            slot + nc, ncells_copy);
@@ -2363,6 +2410,77 @@ static size_t slice_sums_bytes(int64_t nslices)
            ~(size_t)255;
 }
 
+// Widths, offsets and the entry total of up to SLICES_ONE slices in one
+// launch: one block, a thread to a slice (its 64 counts as 16 loads in flight).
+// 123 slices: 3.4 + 3.4 + 7.5 us in the three launches of the general path,
+// 6.4 in this one (two builds of a 15,000-particle dam break: 16.6 -> 5.7);
+// past a thread to a slice the general path's many blocks read the counts
+// faster.  The second block does the second build of a pair.
+#define SLICES_ONE 1024
+struct SlicesOne {
+    const int32_t *counts;  // 16-byte aligned
+    int64_t nd_total;
+    int nslices;
+    int64_t *slice_off, *nnz;
+};
+
+__global__ void __launch_bounds__(SLICES_ONE) k_slices_one(SlicesOne a0, SlicesOne a1)
+{
+    __shared__ longlong2 s_wave[SLICES_ONE / 64];
+    const SlicesOne &a = blockIdx.x ? a1 : a0;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    int m = 0, sum = 0;
+    if (tid < a.nslices) {
+        const int64_t r = (int64_t)tid * 64;
+        if (r + 64 <= a.nd_total) {
+            const int4 *c = (const int4 *)(a.counts + r);
+            int4 v[16];
+#pragma unroll
+            for (int k = 0; k < 16; ++k) v[k] = c[k];
+#pragma unroll
+            for (int k = 0; k < 16; ++k) {
+                m = max(m, max(max(v[k].x, v[k].y), max(v[k].z, v[k].w)));
+                sum += v[k].x + v[k].y + v[k].z + v[k].w;
+            }
+        } else {
+            for (int64_t t = r; t < a.nd_total; ++t) {
+                m = max(m, a.counts[t]);
+                sum += a.counts[t];
+            }
+        }
+    }
+    const int64_t w = 64 * (int64_t)m;
+    int64_t iw = w, is = sum;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int64_t uw = __shfl_up(iw, d, 64), us = __shfl_up(is, d, 64);
+        if (lane >= d) {
+            iw += uw;
+            is += us;
+        }
+    }
+    if (lane == 63) s_wave[wave] = make_longlong2(iw, is);
+    __syncthreads();
+    int64_t before = 0, tw = 0, ts = 0;
+#pragma unroll
+    for (int q = 0; q < SLICES_ONE / 64; ++q) {
+        const longlong2 v = s_wave[q];
+        before += q < wave ? v.x : 0;
+        tw += v.x;
+        ts += v.y;
+    }
+    if (tid < a.nslices) a.slice_off[tid] = before + iw - w;
+    if (tid == 0) {
+        a.slice_off[a.nslices] = tw;
+        *a.nnz = ts;
+    }
+}
+
+static bool slices_one(const int32_t *counts, int64_t nslices)
+{
+    return nslices > 0 && nslices <= SLICES_ONE && ((uintptr_t)counts & 15) == 0;
+}
+
 static int slices_to_offsets(sph_ctx *ctx, int64_t *slice_off, const int64_t *slice_w2,
                              const int64_t *slice_sum, int64_t nslices, int64_t *nnz_dev,
                              size_t scan_scratch_off)
@@ -2453,11 +2571,15 @@ static int count_reset(sph_ctx *ctx, const CellArgs &a, int32_t *counts, int64_t
 }
 
 // slice widths -> offsets (scan); slice totals -> entry total
-static int count_slices(sph_ctx *ctx, const CellArgs &a, const int32_t *counts,
-                        int64_t *slice_off, int64_t *slice_sum, size_t scan_off,
-                        int64_t nd_total)
+static int count_slices(sph_ctx *ctx, const int32_t *counts, int64_t *slice_off,
+                        int64_t *slice_sum, size_t scan_off, int64_t nd_total, int64_t nslices)
 {
-    const int64_t nslices = a.nslices;
+    if (slices_one(counts, nslices)) {
+        const SlicesOne a = {counts, nd_total, (int)nslices, slice_off, slice_sum + nslices};
+        hipLaunchKernelGGL(k_slices_one, dim3(1), dim3(SLICES_ONE), 0, ctx->stream, a, a);
+        SPH_LAUNCH_CHECK(ctx, "k_slices_one");
+        return SPH_OK;
+    }
     hipLaunchKernelGGL(k_slices, dim3(sph_blocks(nslices * 64, NN_THREADS)), dim3(NN_THREADS), 0,
                        ctx->stream, counts, nd_total, nslices, slice_off, slice_sum,
                        slice_sum + nslices + 1);
@@ -2490,7 +2612,7 @@ static int nnps_count(sph_ctx *ctx, CellArgs &a, int64_t ncell_launch, int64_t n
     hipLaunchKernelGGL(count_kern, dim3((unsigned)count_grid(a, ncell_launch)), dim3(CW), 0,
                        ctx->stream, a, counts);
     SPH_LAUNCH_CHECK(ctx, "k_nnps_count");
-    return count_slices(ctx, a, counts, slice_off, slice_sum, scan_off, nd_total);
+    return count_slices(ctx, counts, slice_off, slice_sum, scan_off, nd_total, a.nslices);
 }
 
 static int nnps_fill(sph_ctx *ctx, const CellArgs &a, int64_t ncell_launch, int64_t nd_total,
@@ -2718,9 +2840,16 @@ static int pair_slices(sph_ctx *ctx, NnpsJob &j0, int64_t *sum0, size_t scan0, N
     const int64_t nt0 = (ns0 + SLICE_TILE - 1) / SLICE_TILE;
     const int64_t nt1 = (ns1 + SLICE_TILE - 1) / SLICE_TILE;
     if (ns0 == 0 || ns1 == 0 || nt0 > SLICE_MAX_TILES || nt1 > SLICE_MAX_TILES) {
-        int rc = count_slices(ctx, j0.a, j0.counts, j0.slice_off, sum0, scan0, j0.nd_total);
+        int rc = count_slices(ctx, j0.counts, j0.slice_off, sum0, scan0, j0.nd_total, ns0);
         if (rc) return rc;
-        return count_slices(ctx, j1.a, j1.counts, j1.slice_off, sum1, scan1, j1.nd_total);
+        return count_slices(ctx, j1.counts, j1.slice_off, sum1, scan1, j1.nd_total, ns1);
+    }
+    if (slices_one(j0.counts, ns0) && slices_one(j1.counts, ns1)) {
+        const SlicesOne o0 = {j0.counts, j0.nd_total, (int)ns0, j0.slice_off, sum0 + ns0};
+        const SlicesOne o1 = {j1.counts, j1.nd_total, (int)ns1, j1.slice_off, sum1 + ns1};
+        hipLaunchKernelGGL(k_slices_one, dim3(2), dim3(SLICES_ONE), 0, ctx->stream, o0, o1);
+        SPH_LAUNCH_CHECK(ctx, "k_slices_one");
+        return SPH_OK;
     }
     const SliceArgs s0 = {j0.counts, j0.nd_total, ns0, j0.slice_off, sum0, sum0 + ns0 + 1};
     const SliceArgs s1 = {j1.counts, j1.nd_total, ns1, j1.slice_off, sum1, sum1 + ns1 + 1};
@@ -3532,12 +3661,7 @@ static int nnps_build_varh(sph_ctx *ctx, const sph_grid *grid, const T *d_rec, c
                        (const int64_t *)nullptr, (int32_t *)nullptr,
                        (const int32_t *)c.dcell_of, (const int32_t *)c.cell_ovf);
     SPH_LAUNCH_CHECK(ctx, "k_varh_rows<count>");
-    hipLaunchKernelGGL(k_slices, dim3(sph_blocks(nslices * 64, NN_THREADS)), dim3(NN_THREADS), 0,
-                       ctx->stream, counts, nd_total, nslices, slice_off, slice_sum,
-                       slice_sum + nslices + 1);
-    SPH_LAUNCH_CHECK(ctx, "k_slices");
-    rc = slices_to_offsets(ctx, slice_off, slice_sum + nslices + 1, slice_sum, nslices, nnz_dev,
-                           sums_off + sums_bytes);
+    rc = count_slices(ctx, counts, slice_off, slice_sum, sums_off + sums_bytes, nd_total, nslices);
     if (rc) return rc;
     rc = sph_ensure_pinned(ctx, 3 * sizeof(int64_t));
     if (rc) return rc;
