@@ -691,7 +691,8 @@ typedef struct sph_batch_desc {
      * gives the same results, bit for bit (the per-particle sums keep their
      * order) -- an autotuner picks them by timing */
     int32_t op_threads;       /* threads per block of the fused operator kernels:
-                               * 64, 128 or 256 (default 256) */
+                               * 64, 128 or 256 (default 256, and 64 up to
+                               * 65,536 particles) */
     int32_t op_blocks_per_cu; /* persistent grid of the fused kernels: blocks per
                                * compute unit, each walking a contiguous range of
                                * particle tiles (default 0: one tile per block) */

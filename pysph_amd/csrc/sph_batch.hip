@@ -48,14 +48,19 @@ static unsigned bbox_parts(int nsims)
     return (unsigned)(p < 1 ? 1 : p > BBOX_PARTS ? BBOX_PARTS : p);
 }
 
-// part blockIdx.y of simulation blockIdx.x: value k into box[(s * BBOX_VALS + k) * parts + part]
+// part blockIdx.y of simulation blockIdx.x: value k into box[(s * BBOX_VALS + k) * parts + part];
+// on the way the blocks set the nzero cell counts that k_batch_keys adds to
 __global__ void __launch_bounds__(BT_THREADS)
     k_batch_bbox(const int64_t *__restrict__ sim_off, const double *__restrict__ x,
                  const double *__restrict__ y, const double *__restrict__ z,
-                 const double *__restrict__ h, double *__restrict__ box)
+                 const double *__restrict__ h, double *__restrict__ box,
+                 int32_t *__restrict__ zero, int64_t nzero)
 {
     __shared__ double red[BBOX_VALS][BT_THREADS / 64];
     const int s = blockIdx.x, parts = gridDim.y, part = blockIdx.y;
+    for (int64_t k = ((int64_t)s * parts + part) * BT_THREADS + threadIdx.x; k < nzero;
+         k += (int64_t)gridDim.x * parts * BT_THREADS)
+        zero[k] = 0;
     const int64_t o = sim_off[s], n = sim_off[s + 1] - o;
     const int64_t b = o + n * part / parts, e = o + n * (part + 1) / parts;
     double v[BBOX_VALS];
@@ -91,25 +96,25 @@ __global__ void __launch_bounds__(BT_THREADS)
     }
 }
 
-// The grid of simulation blockIdx.x from its boxes, one per lane
+// The grid of simulation s from its boxes, one per lane of a wavefront
 // (CellManager.compute_cell_size with the Particles defaults: no clamps, 0 ->
 // 1.0).  ncell[s] = cells of the grid; d0 = 0 marks a void simulation, whose
 // particles go to the trash cell.
-__global__ void __launch_bounds__(64)
-    k_batch_grid(const int64_t *__restrict__ sim_off, const double *__restrict__ box, int parts,
-                 double radius_scale, int uniform_h, GridDev *__restrict__ grids,
-                 int64_t *__restrict__ ncell, int32_t *__restrict__ status)
+__device__ void batch_grid(int s, const int64_t *__restrict__ sim_off,
+                           const double *__restrict__ box, int parts, double radius_scale,
+                           int uniform_h, GridDev *grids, int64_t *ncell,
+                           int32_t *__restrict__ status)
 {
-    const int s = blockIdx.x;
+    const int lane = threadIdx.x & 63;
     double v[BBOX_VALS];
 #pragma unroll
     for (int k = 0; k < BBOX_VALS; ++k)
-        v[k] = box[((int64_t)s * BBOX_VALS + k) * parts + min((int)threadIdx.x, parts - 1)];
+        v[k] = box[((int64_t)s * BBOX_VALS + k) * parts + min(lane, parts - 1)];
 #pragma unroll
     for (int k = 0; k < BBOX_VALS; ++k)
 #pragma unroll
         for (int d = BBOX_PARTS / 2; d >= 1; d >>= 1) v[k] = fmin(v[k], __shfl_xor(v[k], d, 64));
-    if (threadIdx.x != 0) return;
+    if (lane != 0) return;
     GridDev g;
     g.tab = nullptr;
     g.key_base = 0;
@@ -150,14 +155,21 @@ __global__ void __launch_bounds__(64)
     ncell[s] = g.d0 ? cells : 0;
 }
 
+__global__ void __launch_bounds__(64)
+    k_batch_grid(const int64_t *__restrict__ sim_off, const double *__restrict__ box, int parts,
+                 double radius_scale, int uniform_h, GridDev *__restrict__ grids,
+                 int64_t *__restrict__ ncell, int32_t *__restrict__ status)
+{
+    batch_grid(blockIdx.x, sim_off, box, parts, radius_scale, uniform_h, grids, ncell, status);
+}
+
 // key_base of every simulation (exclusive sum of the cell counts).  The
 // last key, key_cap - 1, is the trash cell: particles of a void simulation
 // (non-finite values, a grid too large, or no room left in the key space --
 // status |= 2) go there and get no neighbour lists, so a simulation that
 // blew up costs no more than one that did not.
-__global__ void __launch_bounds__(1024)
-    k_batch_key_base(int nsims, const int64_t *__restrict__ ncell, int64_t key_cap,
-                     GridDev *__restrict__ grids, int32_t *__restrict__ status)
+__device__ void batch_key_base(int nsims, const int64_t *ncell, int64_t key_cap, GridDev *grids,
+                               int32_t *__restrict__ status)
 {
     // block-wide exclusive scan of the cells of the live simulations, 1024
     // simulations at a time; a simulation that does not fit becomes void
@@ -200,6 +212,29 @@ __global__ void __launch_bounds__(1024)
         }
         __syncthreads();
     }
+}
+
+__global__ void __launch_bounds__(1024)
+    k_batch_key_base(int nsims, const int64_t *__restrict__ ncell, int64_t key_cap,
+                     GridDev *__restrict__ grids, int32_t *__restrict__ status)
+{
+    batch_key_base(nsims, ncell, key_cap, grids, status);
+}
+
+// both in one launch for a wavefront to a simulation (one simulation: 3.6 +
+// 3.1 -> 4.5 us; with more the grids' latencies would add up in the one block)
+#define GRID_BASE_SIMS 16
+__global__ void __launch_bounds__(1024)
+    k_batch_grid_base(int nsims, const int64_t *__restrict__ sim_off,
+                      const double *__restrict__ box, int parts, double radius_scale,
+                      int uniform_h, int64_t key_cap, GridDev *grids, int64_t *ncell,
+                      int32_t *__restrict__ status)
+{
+    const int s = threadIdx.x >> 6;
+    if (s < nsims)
+        batch_grid(s, sim_off, box, parts, radius_scale, uniform_h, grids, ncell, status);
+    __syncthreads();
+    batch_key_base(nsims, ncell, key_cap, grids, status);
 }
 
 __global__ void __launch_bounds__(BT_THREADS)
@@ -252,13 +287,6 @@ __global__ void __launch_bounds__(BT_THREADS)
     if (act) slot[i] = base + (lane - start);
 }
 
-// more non-empty cells than the list kernels are launched for: status |= 16
-__global__ void k_batch_check_cells(const int32_t *__restrict__ ncell_dev, int64_t max_cells,
-                                    int32_t *__restrict__ status)
-{
-    if (threadIdx.x == 0 && *ncell_dev > max_cells) *status |= 16;
-}
-
 // x = x0 + a * (scale * dt_sim[s]) for the stepped properties (the
 // per-simulation time step of Integrator.step, solver/integrator.py:340-367)
 __global__ void __launch_bounds__(BT_THREADS)
@@ -296,6 +324,7 @@ __global__ void __launch_bounds__(BT_THREADS)
 // part of the sorted order.  NT neighbour records are loaded before their
 // terms are added in list order.
 #define FUSED_MAX_THREADS 256
+#define SMALL_BATCH (256 * FUSED_MAX_THREADS)  // particles
 
 __device__ __forceinline__ void fused_tiles(int64_t ntiles, int64_t &tb, int64_t &te)
 {
@@ -1160,19 +1189,23 @@ int batch_lists(sph_ctx *ctx, const sph_batch_desc *d, const BatchWork &w)
     // -- binning into the per-simulation grids
     const unsigned parts = bbox_parts(d->nsims);
     hipLaunchKernelGGL(k_batch_bbox, dim3(d->nsims, parts), dim3(BT_THREADS), 0, ctx->stream,
-                       d->sim_off, d->x, d->y, d->z, d->h, w.box);
+                       d->sim_off, d->x, d->y, d->z, d->h, w.box, w.slot, d->key_cap + 1);
     SPH_LAUNCH_CHECK(ctx, "k_batch_bbox");
-    hipLaunchKernelGGL(k_batch_grid, dim3(d->nsims), dim3(64), 0, ctx->stream, d->sim_off,
-                       (const double *)w.box, (int)parts, d->radius_scale, d->uniform_h, w.grids,
-                       w.ncell, d->status);
-    SPH_LAUNCH_CHECK(ctx, "k_batch_grid");
-    hipLaunchKernelGGL(k_batch_key_base, dim3(1), dim3(1024), 0, ctx->stream, d->nsims, w.ncell,
-                       d->key_cap, w.grids, d->status);
-    SPH_LAUNCH_CHECK(ctx, "k_batch_key_base");
-    // cell counts into w.slot (sph_bin_sort turns them into w.cell_start)
-    hipLaunchKernelGGL(k_fill_i32, dim3(sph_blocks(d->key_cap + 1, BT_THREADS)),
-                       dim3(BT_THREADS), 0, ctx->stream, w.slot, d->key_cap + 1, 0);
-    SPH_LAUNCH_CHECK(ctx, "k_fill_i32");
+    if (d->nsims <= GRID_BASE_SIMS) {
+        hipLaunchKernelGGL(k_batch_grid_base, dim3(1), dim3(1024), 0, ctx->stream, d->nsims,
+                           d->sim_off, (const double *)w.box, (int)parts, d->radius_scale,
+                           d->uniform_h, d->key_cap, w.grids, w.ncell, d->status);
+        SPH_LAUNCH_CHECK(ctx, "k_batch_grid_base");
+    } else {
+        hipLaunchKernelGGL(k_batch_grid, dim3(d->nsims), dim3(64), 0, ctx->stream, d->sim_off,
+                           (const double *)w.box, (int)parts, d->radius_scale, d->uniform_h,
+                           w.grids, w.ncell, d->status);
+        SPH_LAUNCH_CHECK(ctx, "k_batch_grid");
+        hipLaunchKernelGGL(k_batch_key_base, dim3(1), dim3(1024), 0, ctx->stream, d->nsims,
+                           w.ncell, d->key_cap, w.grids, d->status);
+        SPH_LAUNCH_CHECK(ctx, "k_batch_key_base");
+    }
+    // cell counts in w.slot (sph_bin_sort turns them into w.cell_start)
     hipLaunchKernelGGL(k_batch_keys, dim3(sph_blocks(n, BT_THREADS)), dim3(BT_THREADS), 0,
                        ctx->stream, w.grids, d->sim_of, d->x, d->y, d->z, n, d->key_cap,
                        w.slot, w.cell_of, w.rank, w.key_sim, d->status);
@@ -1182,9 +1215,6 @@ int batch_lists(sph_ctx *ctx, const sph_batch_desc *d, const BatchWork &w)
                       w.slot, w.tmp, trash, 0);
     if (rc) return rc;
     const int32_t *ncell_dev = w.slot + d->key_cap;
-    hipLaunchKernelGGL(k_batch_check_cells, dim3(1), dim3(64), 0, ctx->stream, ncell_dev,
-                       d->max_cells, d->status);
-    SPH_LAUNCH_CHECK(ctx, "k_batch_check_cells");
     // -- sorted records of the fields the operators read (written from the
     // original order into row rank[i]: coalesced reads)
     // in 2D the z and w fields of the records stay zero (the workspace
@@ -1372,7 +1402,12 @@ int batch_eval_stage_fused(sph_ctx *ctx, const sph_batch_desc *d, const BatchWor
 {
     int rc = batch_lists(ctx, d, w);
     if (rc) return rc;
-    const unsigned threads = d->op_threads > 0 ? (unsigned)d->op_threads : FUSED_MAX_THREADS;
+    // one wavefront to a block while 256-row blocks would leave compute units
+    // idle (rollouts of 2,000 to 31,000 particles run 2 to 5 % faster; at
+    // 126,000 the sizes are level)
+    const unsigned threads = d->op_threads > 0    ? (unsigned)d->op_threads
+                             : d->n <= SMALL_BATCH ? 64
+                                                   : FUSED_MAX_THREADS;
     const int64_t ntiles = (d->n + threads - 1) / threads;
     int64_t grid = ntiles;
     if (d->op_blocks_per_cu > 0) {

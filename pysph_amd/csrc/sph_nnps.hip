@@ -2410,6 +2410,30 @@ static size_t slice_sums_bytes(int64_t nslices)
            ~(size_t)255;
 }
 
+// What a batched build reports (status NULL: nothing): bit 0 of *status when
+// the lists need more than cap slots, 16 when the non-empty cells exceed the
+// max_cells the list kernels are launched for; *nnz_acc += nnz (pair count kept
+// on the device)
+struct BatchStatus {
+    int64_t cap, max_cells;
+    const int32_t *ncell_dev;
+    int32_t *status;
+    int64_t *nnz_acc;
+};
+
+__device__ __forceinline__ void batch_status(const BatchStatus &b, int64_t slots, int64_t nnz)
+{
+    const int32_t f = (slots > b.cap ? 1 : 0) | (*b.ncell_dev > b.max_cells ? 16 : 0);
+    if (f) *b.status |= f;
+    if (b.nnz_acc) *b.nnz_acc += nnz;
+}
+
+__global__ void k_nnps_dev_status(const int64_t *__restrict__ slots, const int64_t *__restrict__ nnz,
+                                  BatchStatus b)
+{
+    if (threadIdx.x == 0) batch_status(b, *slots, *nnz);
+}
+
 // Widths, offsets and the entry total of up to SLICES_ONE slices in one
 // launch: one block, a thread to a slice (its 64 counts as 16 loads in flight).
 // 123 slices: 3.4 + 3.4 + 7.5 us in the three launches of the general path,
@@ -2422,6 +2446,7 @@ struct SlicesOne {
     int64_t nd_total;
     int nslices;
     int64_t *slice_off, *nnz;
+    BatchStatus st;
 };
 
 __global__ void __launch_bounds__(SLICES_ONE) k_slices_one(SlicesOne a0, SlicesOne a1)
@@ -2473,6 +2498,7 @@ __global__ void __launch_bounds__(SLICES_ONE) k_slices_one(SlicesOne a0, SlicesO
     if (tid == 0) {
         a.slice_off[a.nslices] = tw;
         *a.nnz = ts;
+        if (a.st.status) batch_status(a.st, tw, ts);
     }
 }
 
@@ -2504,17 +2530,6 @@ static int slices_to_offsets(sph_ctx *ctx, int64_t *slice_off, const int64_t *sl
                        nnz_dev);
     SPH_LAUNCH_CHECK(ctx, "k_sum_i64");
     return sph_scan_exclusive_i64_at(ctx, slice_off, nslices, scan_scratch_off);
-}
-
-// status / totals of a device-side build: bit 0 of *status when the lists
-// need more than cap slots; *nnz_acc += nnz (pair count kept on the device)
-__global__ void k_nnps_dev_status(const int64_t *__restrict__ slots, const int64_t *__restrict__ nnz,
-                                  int64_t cap, int32_t *__restrict__ status,
-                                  int64_t *__restrict__ nnz_acc)
-{
-    if (threadIdx.x != 0) return;
-    if (*slots > cap) *status |= 1;
-    if (nnz_acc) *nnz_acc += *nnz;
 }
 
 // Count pass, slice offsets and totals, then (after the caller's check of
@@ -2572,10 +2587,12 @@ static int count_reset(sph_ctx *ctx, const CellArgs &a, int32_t *counts, int64_t
 
 // slice widths -> offsets (scan); slice totals -> entry total
 static int count_slices(sph_ctx *ctx, const int32_t *counts, int64_t *slice_off,
-                        int64_t *slice_sum, size_t scan_off, int64_t nd_total, int64_t nslices)
+                        int64_t *slice_sum, size_t scan_off, int64_t nd_total, int64_t nslices,
+                        const BatchStatus *st = nullptr)
 {
     if (slices_one(counts, nslices)) {
-        const SlicesOne a = {counts, nd_total, (int)nslices, slice_off, slice_sum + nslices};
+        const SlicesOne a = {counts, nd_total, (int)nslices, slice_off, slice_sum + nslices,
+                             st ? *st : BatchStatus()};
         hipLaunchKernelGGL(k_slices_one, dim3(1), dim3(SLICES_ONE), 0, ctx->stream, a, a);
         SPH_LAUNCH_CHECK(ctx, "k_slices_one");
         return SPH_OK;
@@ -2584,8 +2601,14 @@ static int count_slices(sph_ctx *ctx, const int32_t *counts, int64_t *slice_off,
                        ctx->stream, counts, nd_total, nslices, slice_off, slice_sum,
                        slice_sum + nslices + 1);
     SPH_LAUNCH_CHECK(ctx, "k_slices");
-    return slices_to_offsets(ctx, slice_off, slice_sum + nslices + 1, slice_sum, nslices,
-                             slice_sum + nslices, scan_off);
+    int rc = slices_to_offsets(ctx, slice_off, slice_sum + nslices + 1, slice_sum, nslices,
+                               slice_sum + nslices, scan_off);
+    if (rc || !st) return rc;
+    hipLaunchKernelGGL(k_nnps_dev_status, dim3(1), dim3(64), 0, ctx->stream,
+                       (const int64_t *)(slice_off + nslices),
+                       (const int64_t *)(slice_sum + nslices), *st);
+    SPH_LAUNCH_CHECK(ctx, "k_nnps_dev_status");
+    return SPH_OK;
 }
 
 static int64_t count_grid(const CellArgs &a, int64_t ncell_launch)
@@ -2597,7 +2620,8 @@ static int64_t count_grid(const CellArgs &a, int64_t ncell_launch)
 }
 
 static int nnps_count(sph_ctx *ctx, CellArgs &a, int64_t ncell_launch, int64_t nd_total,
-                      int32_t *counts, int64_t *slice_off, int64_t **nnz_dev)
+                      int32_t *counts, int64_t *slice_off, int64_t **nnz_dev,
+                      const BatchStatus *st = nullptr)
 {
     const CountScratch c = count_scratch(a, ncell_launch, nd_total);
     int rc = sph_ensure_scratch(ctx, c.total);
@@ -2612,7 +2636,7 @@ static int nnps_count(sph_ctx *ctx, CellArgs &a, int64_t ncell_launch, int64_t n
     hipLaunchKernelGGL(count_kern, dim3((unsigned)count_grid(a, ncell_launch)), dim3(CW), 0,
                        ctx->stream, a, counts);
     SPH_LAUNCH_CHECK(ctx, "k_nnps_count");
-    return count_slices(ctx, counts, slice_off, slice_sum, scan_off, nd_total, a.nslices);
+    return count_slices(ctx, counts, slice_off, slice_sum, scan_off, nd_total, a.nslices, st);
 }
 
 static int nnps_fill(sph_ctx *ctx, const CellArgs &a, int64_t ncell_launch, int64_t nd_total,
@@ -2845,8 +2869,8 @@ static int pair_slices(sph_ctx *ctx, NnpsJob &j0, int64_t *sum0, size_t scan0, N
         return count_slices(ctx, j1.counts, j1.slice_off, sum1, scan1, j1.nd_total, ns1);
     }
     if (slices_one(j0.counts, ns0) && slices_one(j1.counts, ns1)) {
-        const SlicesOne o0 = {j0.counts, j0.nd_total, (int)ns0, j0.slice_off, sum0 + ns0};
-        const SlicesOne o1 = {j1.counts, j1.nd_total, (int)ns1, j1.slice_off, sum1 + ns1};
+        const SlicesOne o0 = {j0.counts, j0.nd_total, (int)ns0, j0.slice_off, sum0 + ns0, {}};
+        const SlicesOne o1 = {j1.counts, j1.nd_total, (int)ns1, j1.slice_off, sum1 + ns1, {}};
         hipLaunchKernelGGL(k_slices_one, dim3(2), dim3(SLICES_ONE), 0, ctx->stream, o0, o1);
         SPH_LAUNCH_CHECK(ctx, "k_slices_one");
         return SPH_OK;
@@ -3119,12 +3143,9 @@ int sph_nnps_build_batch(sph_ctx *ctx, const GridDev *grids, const int32_t *sim_
     a.trash = trash;
     a.cells_per_block = cells_per_block;
     int64_t *nnz_dev = nullptr;
-    rc = nnps_count(ctx, a, max_cells, n, counts, slice_off, &nnz_dev);
+    const BatchStatus st = {cap, max_cells, ncell_dev, status, nnz_acc};
+    rc = nnps_count(ctx, a, max_cells, n, counts, slice_off, &nnz_dev, &st);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_nnps_dev_status, dim3(1), dim3(64), 0, ctx->stream,
-                       (const int64_t *)(slice_off + a.nslices), (const int64_t *)nnz_dev, cap,
-                       status, nnz_acc);
-    SPH_LAUNCH_CHECK(ctx, "k_nnps_dev_status");
     return nnps_fill(ctx, a, max_cells, n, counts, slice_off, indices);
 }
 
