@@ -179,6 +179,8 @@ int sph_scatter_sorted2(sph_ctx *ctx, int64_t n, const int32_t *rank, const sph_
                         const sph_prop_list *props2);
 int sph_scatter_sorted_f32(sph_ctx *ctx, int64_t n, const int32_t *rank,
                            const sph_prop_list_f32 *props);
+int sph_scatter_sorted2_f32(sph_ctx *ctx, int64_t n, const int32_t *rank,
+                            const sph_prop_list_f32 *props, const sph_prop_list_f32 *props2);
 
 /* Neighbour lists of FixedDestNbrParticleLocator (base/nnps.pyx:458-621)
  * in SORTED space, stored as sliced ELLPACK with 64-row slices (SELL-64):

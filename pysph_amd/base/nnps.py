@@ -119,8 +119,8 @@ class _Bins:
         self.pending = None
         self.rec = torch.zeros((max(n, 1), REC), dtype=dtype, device=device)
         self.shadow_ver = {}
-        # compact sorted (x, y, z, m) rows (FP64 only): the neighbour gathers
-        # of density and momentum touch fewer cache lines than in the records
+        # compact sorted (x, y, z, m) rows: the neighbour gathers of density
+        # touch fewer cache lines than in the records
         self.pm = None
         self.pm_ver = {}
         self.stamp = 0
@@ -424,11 +424,13 @@ class CellManager:
                 pl.dst[k] = b.field_ptr(p)
             # original order -> sorted rows by rank: coalesced reads of every
             # field (the gather by perm reads one cache line per lane and field)
-            pm = self._pm_props(array, b) if not single else None
+            pm = self._pm_props(array, b)
             with profiling.region("gather_sorted"):
                 if pm is not None:  # the compact rows in the same pass
-                    ctx.check(ctx.lib.sph_scatter_sorted2(ctx.handle, b.n, _lib.ptr(b.rank),
-                                                          ctypes.byref(pl), ctypes.byref(pm[0])))
+                    scatter = (ctx.lib.sph_scatter_sorted2_f32 if single
+                               else ctx.lib.sph_scatter_sorted2)
+                    ctx.check(scatter(ctx.handle, b.n, _lib.ptr(b.rank), ctypes.byref(pl),
+                                      ctypes.byref(pm[0])))
                 else:
                     scatter = (ctx.lib.sph_scatter_sorted_f32 if single
                                else ctx.lib.sph_scatter_sorted)
@@ -448,36 +450,35 @@ class CellManager:
         stale = [q for q in PM_FIELDS if b.pm_ver.get(q) != array.version(q)]
         if not stale:
             return None
-        pl = _lib.PropList()
+        pl = _lib.PropListF32() if self.precision == "single" else _lib.PropList()
         pl.nprops = len(stale)
         pl.dst_stride = 4
-        base = b.pm.data_ptr()
+        base, size = b.pm.data_ptr(), b.pm.element_size()
         for k, q in enumerate(stale):
             src = array.get_carray(q)
             if src is None or src.dtype != torch.float64:
                 raise TypeError(f"property {q} of {array.name} must be float64")
             pl.src[k] = _lib.ptr(src)
-            pl.dst[k] = base + 8 * PM_FIELDS.index(q)
+            pl.dst[k] = base + size * PM_FIELDS.index(q)
         return pl, stale
 
     def posmass(self, array):
-        """The compact sorted (x, y, z, m) rows of `array` (4 doubles per
-        particle, rows in record order) with stale fields refreshed, or None
-        in single precision (the float records are read instead)."""
-        if self.precision == "single":
-            return None
+        """The compact sorted (x, y, z, m) rows of `array` (4 values of the
+        records' type per particle, rows in record order) with stale fields
+        refreshed."""
         self.update()
         b = self.bins[array.name]
         if b.pm is None or b.pm.shape[0] != max(b.n, 1):
-            b.pm = torch.empty((max(b.n, 1), 4), dtype=torch.float64, device=b.device)
+            b.pm = torch.empty((max(b.n, 1), 4), dtype=self.rec_dtype, device=b.device)
             b.pm_ver = {}
         pm = self._pm_props(array, b)
         if pm is not None:
             ctx = self._ctx()
             pl, stale = pm
             with profiling.region("gather_sorted"):
-                ctx.check(ctx.lib.sph_scatter_sorted(ctx.handle, b.n, _lib.ptr(b.rank),
-                                                     ctypes.byref(pl)))
+                scatter = (ctx.lib.sph_scatter_sorted_f32 if self.precision == "single"
+                           else ctx.lib.sph_scatter_sorted)
+                ctx.check(scatter(ctx.handle, b.n, _lib.ptr(b.rank), ctypes.byref(pl)))
             for q in stale:
                 b.pm_ver[q] = array.version(q)
         return b.pm

@@ -83,8 +83,30 @@ __device__ __forceinline__ void tait_point(const TaitArgs<T> &E, int64_t t, int3
 // ---------------------------------------------------------------------------
 // SPHRho (rho_term in sph_terms.h)
 // ---------------------------------------------------------------------------
-// one SELL-64 row of SPHRho, summed from 0 in list order
-template <bool UH, bool SHORT, typename T>
+// the (x, y) and (z, m) of source j: from the compact rows (PM, float: one
+// 16-byte load; in FP64 two, like the record's) or the record
+template <bool PM, typename T, typename P>
+__device__ __forceinline__ void rho_source(const T *__restrict__ spm, const T *__restrict__ srec,
+                                           int32_t j, P &a, P &b)
+{
+    if constexpr (PM && sizeof(T) == sizeof(float)) {
+        const float4 v = reinterpret_cast<const float4 *>(spm)[j];
+        a.x = v.x;
+        a.y = v.y;
+        b.x = v.z;
+        b.y = v.w;
+    } else {
+        const P *sp = pm2(spm, srec, j);
+        a = sp[0];
+        b = sp[1];
+    }
+}
+
+// one SELL-64 row of SPHRho, summed from 0 in list order.  PM: float, and the
+// compact rows are there: the gathers set the pace, and one 16-byte load from
+// rows of 16 bytes takes less of it than two 8-byte loads from rows of 48 (1M
+// lattice 219 -> 144 us; 16-byte loads from the records gained nothing).
+template <bool UH, bool SHORT, bool PM, typename T>
 __device__ __forceinline__ T rho_row(int dim, T xa, T ya, T za, T ha, T facA,
                                      const int32_t *__restrict__ row, int32_t e,
                                      const T *__restrict__ srec, const T *__restrict__ spm)
@@ -105,9 +127,7 @@ __device__ __forceinline__ T rho_row(int dim, T xa, T ya, T za, T ha, T facA,
             j[u] = __builtin_nontemporal_load(row + ((int64_t)(k + u) << 6));
 #pragma unroll
         for (int u = 0; u < DENS_NT; ++u) {
-            const P *sp = pm2(spm, srec, j[u]);
-            a[u] = sp[0];
-            b[u] = sp[1];
+            rho_source<PM>(spm, srec, j[u], a[u], b[u]);
             hb[u] = UH ? ha : srec[(int64_t)j[u] * SPH_REC + SPH_R_H];
         }
 #pragma unroll
@@ -116,9 +136,10 @@ __device__ __forceinline__ T rho_row(int dim, T xa, T ya, T za, T ha, T facA,
     }
     for (; k < e; ++k) {
         const int32_t j = __builtin_nontemporal_load(row + ((int64_t)k << 6));
-        const P *sp = pm2(spm, srec, j);
+        P a, b;
+        rho_source<PM>(spm, srec, j, a, b);
         const T hb = UH ? ha : srec[(int64_t)j * SPH_REC + SPH_R_H];
-        nr += rho_term<UH, T, P, SHORT>(dim, xa, ya, za, ha, facA, sp[0], sp[1], hb, invA);
+        nr += rho_term<UH, T, P, SHORT>(dim, xa, ya, za, ha, facA, a, b, hb, invA);
     }
     return nr;
 }
@@ -162,8 +183,15 @@ __global__ void __launch_bounds__(OP_THREADS)
         const T facA = sph_h_dim(ha, dim) * sph_cubic_fac1<T>(dim);
         for (int s = 0; s < L.nsrc; ++s) {
             const int32_t *row = L.indices[s] + L.slice_off[s][t >> 6] + (t & 63);
-            val = val + rho_row<h_one<HM, T>, h_short<HM, T>, T>(dim, xa, ya, za, ha, facA, row,
-                                                                 e[s], L.srec[s], L.spm[s]);
+            constexpr bool F32 = sizeof(T) == sizeof(float);
+            T r;
+            if (F32 && L.spm[s])
+                r = rho_row<h_one<HM, T>, h_short<HM, T>, F32, T>(dim, xa, ya, za, ha, facA, row,
+                                                                  e[s], L.srec[s], L.spm[s]);
+            else
+                r = rho_row<h_one<HM, T>, h_short<HM, T>, false, T>(dim, xa, ya, za, ha, facA, row,
+                                                                    e[s], L.srec[s], L.spm[s]);
+            val = val + r;
         }
     }
     rho[i] = val;

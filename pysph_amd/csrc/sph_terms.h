@@ -168,7 +168,8 @@ static int src_lists(sph_ctx *ctx, const char *name, const sph_sources *src, Src
         L->slice_off[s] = src->slice_off[s];
         L->indices[s] = src->indices[s];
         L->srec[s] = (const T *)src->s_rec[s];
-        L->spm[s] = (const T *)src->s_pm[s];
+        // read as 16-byte words: rows that are not aligned to them are left out
+        L->spm[s] = ((uintptr_t)src->s_pm[s] & 15) == 0 ? (const T *)src->s_pm[s] : nullptr;
     }
     return SPH_OK;
 }
