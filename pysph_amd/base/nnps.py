@@ -934,9 +934,16 @@ class VarHNbrParticleLocator(FixedDestNbrParticleLocator):
         slots = ctypes.c_int64(0)
         nnz = ctypes.c_int64(0)
         p = _lib.ptr
-        # a bound of every h now (h may have been written since the binning)
-        max_h = max(float(a.get_carray("h")[:a.get_number_of_particles()].max())
-                    for a in (dst, src) if a.get_number_of_particles() > 0)
+        # a bound of every h now: the grid's, when it covers these arrays alone
+        # and no h was written since it was built; else two reductions and
+        # read-backs (493,000 particles: 1.12 ms for binning, lists and
+        # density with them, 1.07 without)
+        if all(a is dst or a is src for a in cm.arrays_to_bin) and cm.grid.max_h >= 0.0 and \
+                all(cm._h_versions.get(a.name) == a.version("h") for a in (dst, src)):
+            max_h = cm.grid.max_h
+        else:
+            max_h = max(float(a.get_carray("h")[:a.get_number_of_particles()].max())
+                        for a in (dst, src) if a.get_number_of_particles() > 0)
 
         # the destination's non-empty cells: counted on the device after the
         # first binning (the launch bound then bounds the count)
