@@ -14,6 +14,7 @@
 #include <string.h>
 
 #include "sph_internal.h"
+#include "sph_count.h"
 
 #define NN_THREADS 256
 
@@ -1517,8 +1518,11 @@ __device__ void nnps_cell_fill(const CellArgs &a, int64_t w, int32_t *__restrict
 // constant and two of each coordinate move the value by less than
 // 44 * 2^-24 M^2.  The band is 64 * 2^-24 M^2 (1.5e-5 cells^2: one 64 x 16
 // tile in 150 of a disordered set holds such a pair).  A chunk with a
-// coordinate outside M (a particle clamped into the grid, a non-finite one)
-// is decided by the predicate throughout.
+// candidate outside M (a particle clamped into the grid, a non-finite one) and
+// a group with such a destination or a radius above the reach are decided by
+// the predicate throughout, for the candidates that exist (sph_count.h).  A
+// state that turned non-finite is reported one binning later, so the lists
+// built from it are used and must hold sources that exist.
 //
 // Candidate 16 g + 4 b + r of a chunk is row 4 g + r of product b, so lane
 // 16 g + j ends with 16 consecutive candidates of destination j: its signs,
@@ -1535,9 +1539,6 @@ __device__ void nnps_cell_fill(const CellArgs &a, int64_t w, int32_t *__restrict
 // the next chunk's data ahead cost the registers of two wavefronts and were
 // slower on the 3D cells (220 to 250 us).
 #define NN_WIN 512                   // candidates listed in LDS at a time
-#define NN_BAND (64.0f * 0x1p-24f)   // times M^2
-#define NN_FAR 1e30f                 // value of an absent candidate or destination
-
 #define NN_COUNT_WAVES 6              // wavefronts per SIMD the count kernels are compiled for
 
 typedef float nn_f32x4 __attribute__((ext_vector_type(4)));
@@ -1639,10 +1640,11 @@ __device__ __forceinline__ void nnps_cell_count(const CellArgs &a, int64_t w, in
             const float x = (float)((double)dr[SPH_R_X] - ox) * inv,
                         y = (float)((double)dr[SPH_R_Y] - oy) * inv,
                         z = (float)((double)dr[SPH_R_Z] - oz) * inv;
-            odd = !(fmaxf(fmaxf(fabsf(x), fabsf(y)), fabsf(z)) <= lim);
             const double rr = (double)radius * inv_cs;
+            odd = !nn_regular(x, y, z, (float)rr, lim);
             dv = make_float4(-2.0f * x, -2.0f * y, -2.0f * z,
                              (float)((double)x * x + (double)y * y + (double)z * z - rr * rr));
+            if (odd) dv = make_float4(0.f, 0.f, 0.f, 0.f);  // the products decide nothing
         }
         wave_lds_order();  // the last group's reads are done
         *reinterpret_cast<float4 *>(&S.d[4 * lane]) = dv;
@@ -1688,7 +1690,7 @@ __device__ __forceinline__ void nnps_cell_count(const CellArgs &a, int64_t w, in
                         v.x = (float)((double)sr[SPH_R_X] - ox) * inv;
                         v.y = (float)((double)sr[SPH_R_Y] - oy) * inv;
                         v.z = (float)((double)sr[SPH_R_Z] - oz) * inv;
-                        far = !(fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fabsf(v.z)) <= lim);
+                        far = !nn_inside(v.x, v.y, v.z, lim);
                         v.w = fmaf(v.x, v.x, fmaf(v.y, v.y, v.z * v.z));
                     }
                     const bool all = odd_d || __builtin_amdgcn_ballot_w64(far) != 0;
@@ -1719,23 +1721,10 @@ __device__ __forceinline__ void nnps_cell_count(const CellArgs &a, int64_t w, in
                         }
                         if (all || __builtin_amdgcn_ballot_w64(near < band)) {
                             // the undecided pairs by the predicate itself
-                            const int32_t left = wn - (c0 + 16 * quarter);
-                            uint32_t ask = left >= 16 ? 0xffffu : left > 0 ? (1u << left) - 1u : 0u;
-                            if (C == NN_FAR) ask = bits = 0;  // no such destination
-                            if (!all) {
-                                uint32_t in = 0;
-#pragma unroll
-                                for (int e = 15; e >= 0; --e)
-                                    in = 2 * in + (fabsf(D[e >> 2][e & 3]) < band);
-                                ask &= in;
-                            }
-                            while (ask) {
-                                const int e = __ffs(ask) - 1;
-                                ask &= ask - 1;
-                                const bool hit = nnps_hit<T>(srec, drec, T(a.rs),
-                                                             S.p[c0 + 16 * quarter + e], g0 + j);
-                                bits = (bits & ~(1u << e)) | ((uint32_t)hit << e);
-                            }
+                            const int q0 = c0 + 16 * quarter;
+                            bits = nn_decide(bits, D, band, all, C == NN_FAR, wn - q0, [&](int e) {
+                                return nnps_hit<T>(srec, drec, T(a.rs), S.p[q0 + e], g0 + j);
+                            });
                         }
                         S.n[CW * t + lane] += __popc(bits);
                         if (cidx < a.maxch && j < gn)
