@@ -24,6 +24,15 @@ __host__ __device__ __forceinline__ bool nn_regular(float x, float y, float z, f
     return nn_inside(x, y, z, lim) && fabsf(radius) <= lim;
 }
 
+// Cell sizes whose float reciprocal, and coordinates over it, keep their 24
+// bits, and whose squares neither underflow nor overflow in the float
+// predicate: the band's assumptions.  Other grids are decided by the predicate
+// throughout.
+__host__ __device__ __forceinline__ bool nn_cell_size(double cs)
+{
+    return cs >= 0x1p-60 && cs <= 0x1p60;
+}
+
 // bits 0..15: which of a lane's candidates exist, `left` of them or more
 __host__ __device__ __forceinline__ uint32_t nn_present(int32_t left)
 {

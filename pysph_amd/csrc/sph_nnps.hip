@@ -1518,9 +1518,10 @@ __device__ void nnps_cell_fill(const CellArgs &a, int64_t w, int32_t *__restrict
 // constant and two of each coordinate move the value by less than
 // 44 * 2^-24 M^2.  The band is 64 * 2^-24 M^2 (1.5e-5 cells^2: one 64 x 16
 // tile in 150 of a disordered set holds such a pair).  A chunk with a
-// candidate outside M (a particle clamped into the grid, a non-finite one) and
-// a group with such a destination or a radius above the reach are decided by
-// the predicate throughout, for the candidates that exist (sph_count.h).  A
+// candidate outside M (a particle clamped into the grid, a non-finite one), a
+// group with such a destination or a radius above the reach, and cells of
+// less than 2^-60 or more than 2^60 are decided by the predicate throughout,
+// for the candidates that exist (sph_count.h).  A
 // state that turned non-finite is reported one binning later, so the lists
 // built from it are used and must hold sources that exist.
 //
@@ -1796,7 +1797,8 @@ __device__ __forceinline__ void count_cells(const CellArgs &a, int32_t *__restri
                 cell_coords<T>(a, gl, ds, cx, cy, cz);
             }
         }
-        const double inv = 1.0 / gl.cs;
+        // (a NaN sends every pair of such a cell to the predicate)
+        const double inv = nn_cell_size(gl.cs) ? 1.0 / gl.cs : NAN;
         uint64_t todo = __builtin_amdgcn_ballot_w64(act);
         while (todo) {
             const int l = __ffsll((unsigned long long)todo) - 1;
