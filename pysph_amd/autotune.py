@@ -30,8 +30,9 @@ SPACE = {
     "staged": (0, 1),
 }
 
-DEFAULT = {"cells_per_block": 0, "op_threads": 256, "op_blocks_per_cu": 0, "nbr_tile": 4,
-           "persistent": 0, "staged": 0}
+# where the walk starts: what an untuned batch runs (0: the library's own choice,
+# which depends on the batch's size)
+DEFAULT = {k: 0 for k in TUNE_FIELDS}
 
 
 def cache_path():
