@@ -10,9 +10,13 @@ keep their order -- so the tuner may pick any of them by speed alone.
 ``autotune`` times real steps of the batch itself (the state is restored
 afterwards) and walks the parameters one at a time (coordinate descent,
 ``rounds`` passes), keeping the fastest value of each.  The choice is cached
-per device, dimension, precision and batch size in a JSON file, so a later
-batch of the same shape starts from it without timing again.
+per device, dimension, precision, batch size and kernel sources in a JSON file,
+so a later batch of the same shape starts from it without timing again, and
+kernels that changed are timed anew.
 """
+import functools
+import glob
+import hashlib
 import json
 import os
 import time
@@ -41,13 +45,29 @@ def cache_path():
     return os.path.join(base, "autotune.json")
 
 
+CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
+
+
+@functools.lru_cache(maxsize=None)
+def _kernels(csrc):
+    """Digest of the kernels' sources: what was the fastest shape for others
+    need not be for these."""
+    digest = hashlib.sha256()
+    for path in sorted(glob.glob(os.path.join(csrc, "*.hip")) +
+                       glob.glob(os.path.join(csrc, "*.h"))):
+        with open(path, "rb") as f:
+            digest.update(f.read())
+    return digest.hexdigest()[:12]
+
+
 def signature(sim):
-    """Cache key: device, dimension, precision, simulations and particles
-    (rounded to 2 significant digits)."""
+    """Cache key: device, dimension, precision, simulations, particles (rounded
+    to 2 significant digits) and kernels."""
     name = torch.cuda.get_device_name(sim.device).replace(" ", "_")
     n = sim.n
     mag = 10 ** max(0, len(str(n)) - 2)
-    return f"{name}/dim{sim.dim}/{sim.precision}/sims{sim.nsims}/n{round(n / mag) * mag}"
+    return (f"{name}/dim{sim.dim}/{sim.precision}/sims{sim.nsims}/n{round(n / mag) * mag}"
+            f"/{_kernels(CSRC)}")
 
 
 def _load_cache(path):

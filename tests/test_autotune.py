@@ -44,3 +44,14 @@ def test_walk_starts_from_what_an_untuned_batch_runs(batch, monkeypatch):
     res = autotune.autotune(batch, space={"nbr_tile": (1, 2, 4)})
     assert res["trials"][0][0] == untuned
     assert res["tuning"] == dict(untuned, nbr_tile=2) == batch.tuning()
+
+
+def test_shapes_tuned_for_other_kernels_are_not_used(batch, monkeypatch, tmp_path):
+    monkeypatch.setattr(autotune, "time_steps", lambda sim, steps, dt: 1.0)
+    space = {"nbr_tile": (1, 2)}
+    assert not autotune.autotune(batch, space=space)["cached"]
+    assert autotune.autotune(_Batch(), space=space)["cached"]
+    (tmp_path / "csrc").mkdir()
+    (tmp_path / "csrc" / "other.hip").write_text("// other kernels")
+    monkeypatch.setattr(autotune, "CSRC", str(tmp_path / "csrc"), raising=False)
+    assert not autotune.autotune(_Batch(), space=space)["cached"]
