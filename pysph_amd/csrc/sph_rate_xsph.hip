@@ -12,6 +12,7 @@
 
 #define RX_THREADS 256
 #define RX_NT 4  // neighbour records in flight per lane
+#define XSPH_SMALL (64 * 1024)  // destinations up to which k_xsph takes the short sequences
 
 // ---------------------------------------------------------------------------
 // SPHDensityRate (sph/funcs/density_funcs.pyx:116-164; hks and the kernel
@@ -235,10 +236,13 @@ static int xsph(sph_ctx *ctx, int dim, int64_t nd_total, int64_t nd_real, const 
     int rc = check_list_op<T>(ctx, "sph_xsph", dim, nd_total, nd_real, d_perm, counts,
                               slice_off, d_rec, s_rec, ox);
     if (rc || nd_total == 0) return rc;
-    // the gathers set the pace of a large array, and the short sequences' longer
-    // live ranges cost more than they save there (512,000 fluid particles 288
-    // us, 317 with them)
-    auto kern = uniform_h == H_SHORT && nd_total <= 256 * 1024 ? k_xsph<H_SHORT, T>
+    // The short sequences pay while the wavefronts wait for their own
+    // arithmetic, and cost more in longer live ranges than they save once the
+    // gathers set the pace.  IEEE -> short, split dam break: 15,000 fluid
+    // particles 40.6 -> 37.5 us, 64,000 50.6 -> 49.6, 125,000 75.0 -> 80.8,
+    // 221,000 147 -> 158, 260,000 148 -> 161; 2D drop: 20,000 19.5 -> 18.6,
+    // 64,000 22.1 -> 21.0, 126,000 31.0 -> 31.1, 242,000 42.4 -> 43.8.
+    auto kern = uniform_h == H_SHORT && nd_total <= XSPH_SMALL ? k_xsph<H_SHORT, T>
                 : uniform_h          ? k_xsph<H_ONE, T>
                                      : k_xsph<H_READ, T>;
     hipLaunchKernelGGL(kern, dim3(sph_blocks(nd_total, RX_THREADS)), dim3(RX_THREADS), 0,
