@@ -766,9 +766,10 @@ int sph_batch_vjp(sph_ctx *ctx, const sph_batch_desc *d, const double *abar_u,
 int sph_batch_rk2_step_kept(sph_ctx *ctx, const sph_batch_desc *d, double dt, void *work2);
 
 /* Reverse of such a step, X1 = X0 + dt/2 F(X0), X2 = X0 + dt F(X1) with
- * F = (u, a): bar (device, rows x y (z) u v (w) of n) holds X2's adjoint and is
- * replaced by X0's; x1 (the same size) receives X1's; the alpha terms are
- * added to *alpha_bar (device scalar). */
+ * F = (u, a) and one dt for all (SPH_EINVAL when the descriptor has dt_sim):
+ * bar (device, rows x y (z) u v (w) of n) holds X2's adjoint and is replaced
+ * by X0's; x1 (the same size) receives X1's; the alpha terms are added to
+ * *alpha_bar (device scalar). */
 int sph_batch_rk2_vjp(sph_ctx *ctx, const sph_batch_desc *d, double dt, void *work2, double *bar,
                       double *x1, double *alpha_bar);
 

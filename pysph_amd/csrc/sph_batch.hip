@@ -1624,6 +1624,7 @@ extern "C" int sph_batch_rk2_vjp(sph_ctx *ctx, const sph_batch_desc *d, double d
     if (rc) return rc;
     SPH_REQUIRE(ctx, bar && x1 && alpha_bar, "sph_batch_rk2_vjp: null argument");
     SPH_REQUIRE(ctx, !d->f32, "sph_batch_rk2_vjp: the reverse mode runs in FP64 only");
+    SPH_REQUIRE(ctx, !d->dt_sim, "sph_batch_rk2_vjp: one time step for all simulations");
     const int64_t n = d->n;
     double *b[6], *y[6];  // rows x y (z) u v (w)
     for (int c = 0; c < 6; ++c) b[c] = y[c] = nullptr;
