@@ -369,10 +369,12 @@ int sph_nnps_export(sph_ctx *ctx, int64_t nd_real, const int32_t *d_rank,
  * be NULL) receives the same values at out_s[t * out_s_stride].
  * uniform_h = 1 asserts that every destination and source particle has the
  * same h (then (h_i+h_j)/2 == h_i exactly and h_j is not read).
- * uniform_h = 2 asserts that and that h lies in [2^-100, 2^100]: the FP64
- * kernels may then take square roots and divisions without the steps for
- * extreme exponents (the same values).  The float and staged kernels take 2
- * as 1. */
+ * uniform_h = 2 asserts that, that h lies in [2^-100, 2^100] and that the
+ * squared distance of every list entry is finite: the FP64 kernels may then
+ * take square roots and divisions without the steps for extreme exponents.
+ * W is the same value, and the gradient factor the same but for operands of
+ * a chance of about 2^-90, where it may be an ulp off.  The float and staged
+ * kernels take 2 as 1. */
 int sph_summation_density(sph_ctx *ctx, int dim, int64_t nd_total, int64_t nd_real,
                           const int32_t *d_perm, const int32_t *counts,
                           const int64_t *slice_off, const int32_t *indices,

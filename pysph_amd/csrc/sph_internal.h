@@ -301,7 +301,7 @@ __device__ __forceinline__ T sph_cubic_gfac_fac(T rx, T ry, T rz, T h, T fac, T 
 }
 
 // ------------------------------------------------------------------------
-// The same values with fewer operations, for rows whose destination's h
+// W and its gradient with fewer operations, for rows whose destination's h
 // (every pair's h) passes sph_short_h.
 //
 // An IEEE FP64 square root or division is a reciprocal estimate, two
@@ -316,8 +316,19 @@ __device__ __forceinline__ T sph_cubic_gfac_fac(T rx, T ry, T rz, T h, T fac, T 
 //     2^-250 gives q <= 2^-150, where W's polynomial is exactly 1 and the
 //     gradient factor is 0 (q <= 1e-14).
 // The gradient's division by h*r takes its reciprocal estimate from the
-// root's refinement (1/r to about 2^-48) times 1/h instead of a reciprocal
-// instruction; one refinement leaves it as close as the IEEE sequence's own.
+// root's refinement (1/r to 2^-47.7, the worst of 4.3e9 samples) times 1/h
+// instead of a reciprocal instruction.  One refinement makes it the reciprocal
+// of the denominator to about 2^-95 before its rounding, so it is the
+// correctly rounded one unless that lies this close to a rounding boundary
+// (about one denominator in 2^41); from the correctly rounded reciprocal the
+// last step gives the IEEE quotient (Markstein's theorem), and from its
+// neighbour too unless the quotient lies within 2^-52 of its last place from
+// a midpoint.  The square root and q are the IEEE ones; so is the gradient
+// factor but for such a denominator and quotient at once, where it may be an
+// ulp off.  No difference in 4.3e9 random pairs.
+//
+// The pairs' r^2 must be finite (an infinite one gives NaN, not 0): the lists
+// hold no others.
 // q > 2 needs no test: 2 - q is clamped at 0, and a term of +-0 leaves a sum
 // that started from +0 unchanged.
 // ------------------------------------------------------------------------

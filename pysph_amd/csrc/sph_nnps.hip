@@ -1262,13 +1262,11 @@ __device__ __forceinline__ uint64_t wave_bcast_u64(uint64_t v, int l)
     return ((uint64_t)hi << 32) | lo;
 }
 
-// FILL = false: count pass.  Runs the distance tests, writes counts[t], the
-//   64-bit hit mask of every (destination, candidate chunk) pair to a.masks,
-//   the cell of every destination and the source of each candidate.  Cells
-//   whose stencil needs more than one batch or more than NN_MAXCH chunks are
-//   flagged in a.cell_ovf.
-// FILL = true: writes the SELL-64 rows of the flagged cells only (the other
-//   cells are written by k_nnps_fill_slices from the masks).
+// The count pass writes counts[t], the 64-bit hit mask of every (destination,
+// candidate chunk) pair to a.masks, the cell of every destination and the
+// source of each candidate.  Cells whose stencil needs more than one batch or
+// more than NN_MAXCH chunks are flagged in a.cell_ovf: nnps_cell_fill writes
+// their rows, k_nnps_fill_slices those of the other cells from the masks.
 template <typename T> struct Quad;
 template <> struct Quad<double> {
     using type = double4;
@@ -1512,18 +1510,20 @@ __device__ void nnps_cell_fill(const CellArgs &a, int64_t w, int32_t *__restrict
 // The signs are exact: coordinates are taken relative to the destination
 // cell's centre (double subtraction), rounded to float and scaled to cells,
 // and a value within NN_BAND of zero is decided by the reference's own FP64
-// (or float) predicate.  With every coordinate below M = reach + 1 cells the
-// partial sums stay below 3.25 M^2: eight float roundings of them (four
-// products and four additions, in any order), three of |c|^2, one of the
-// constant and two of each coordinate move the value by less than
-// 44 * 2^-24 M^2.  The band is 64 * 2^-24 M^2 (1.5e-5 cells^2: one 64 x 16
-// tile in 150 of a disordered set holds such a pair).  A chunk with a
-// candidate outside M (a particle clamped into the grid, a non-finite one), a
-// group with such a destination or a radius above the reach, and cells of
-// less than 2^-60 or more than 2^60 are decided by the predicate throughout,
-// for the candidates that exist (sph_count.h).  A
-// state that turned non-finite is reported one binning later, so the lists
-// built from it are used and must hold sources that exist.
+// (or float) predicate.  Let u = 2^-24 and every coordinate and the radius be
+// below M = reach + 1 cells.  Of a pair whose value is near zero, c and d
+// differ by at most the radius, so the value moves by less than 16 u M^2 for
+// the coordinates (two roundings each, and the scale's), 9 for the three of
+// |c|^2, 3 for the constant, 9 for the four products and 12 for the four
+// additions in any order: 49 u M^2, and in single precision the predicate is
+// itself off by 6.  The band is 64 u M^2 (1.5e-5 cells^2: one 64 x 16 tile in
+// 150 of a disordered set holds such a pair).  A chunk with a candidate
+// outside M (a particle clamped into the grid, a non-finite one), a group with
+// such a destination or a radius above the reach, and cells of less than 2^-60
+// or more than 2^60 are decided by the predicate throughout, for the
+// candidates that exist (sph_count.h).  A state that turned non-finite is
+// reported one binning later, so the lists built from it are used and must
+// hold sources that exist.
 //
 // Candidate 16 g + 4 b + r of a chunk is row 4 g + r of product b, so lane
 // 16 g + j ends with 16 consecutive candidates of destination j: its signs,

@@ -23,9 +23,10 @@
 #define MOM_NT 4
 #endif
 // the short sequences pay where a few wavefronts wait for their own
-// arithmetic (15,000 fluid particles 75 -> 63 us a launch, 125,000 in 2D 27
-// -> 21 us), with three records in flight; where the gathers set the pace they
-// do not (1M dam break 650 -> 684 us): up to MOM_SMALL destinations
+// arithmetic, with three records in flight; where the gathers set the pace they
+// do not.  IEEE -> short a launch: dam break of 15,000 fluid particles 85 -> 68
+// us, 64,000 96 -> 83, 125,000 111 -> 106, 260,000 220 -> 215, 1M 650 -> 684; 2D
+// drop of 126,000 36 -> 33, 242,000 49 -> 46: up to MOM_SMALL destinations
 #ifndef MOM_NT_SHORT
 #define MOM_NT_SHORT 3
 #endif
